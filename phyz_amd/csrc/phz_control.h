@@ -46,6 +46,8 @@ struct ObsArgs {
   const void* v;  // [nv][stride] T
   void* kin;      // [nb * XF_STRIDE][stride] T, written when write_kin
   float* obs;     // [n_in][stride] f32, the history row of this control step, written when write_obs
+  void* hq;       // state-history rows ([nq][stride], [nv][stride] T) of the control step before,
+  void* hv;       // whose final state is the one read here; null to record nothing
   int nworld;
   int stride;
   int write_kin;
@@ -160,6 +162,12 @@ template <class M, class O, class T> __device__ __forceinline__ void obs_world(c
   for (int j = 0; j < M::NQ; j++) q[j] = gq[j * S + w];
 #pragma unroll
   for (int j = 0; j < M::NV; j++) v[j] = gv[j * S + w];
+  if (a.hq != nullptr) {
+#pragma unroll
+    for (int j = 0; j < M::NQ; j++) ((T*)a.hq)[j * S + w] = q[j];
+#pragma unroll
+    for (int j = 0; j < M::NV; j++) ((T*)a.hv)[j * S + w] = v[j];
+  }
   FKState<M, T> f;
   fk_all<M, T>(q, v, f);
   if (a.write_kin) {
