@@ -11,14 +11,17 @@
 //               FK in registers; the FK readout rows and the observation row
 //               are stored structure-of-arrays ([j][stride]) so a wave's
 //               stores coalesce.
-//   phz_policy  one wave per 16*CB worlds. The three MLP layers run on f32
-//               MFMA (v_mfma_f32_16x16x4f32) with the weights as the A
-//               operand and the activations as the B operand, so a layer's
-//               16x16 output tiles are already laid out as the next layer's
-//               B fragments: hidden activations never leave registers. Only
-//               the per-world prologue (input noise) and epilogue (Gaussian
-//               sample, log-prob, PD targets) go through LDS, because each
-//               world's random stream is sequential and lives in one lane.
+//   phz_policy  one wave per 16*CB worlds. The three MLP layers run on MFMA
+//               with the weights as the A operand and the activations as the
+//               B operand, so a layer's 16x16 output tiles are already laid
+//               out as the next layer's B fragments: hidden activations never
+//               leave registers. The first layer is f32 (16x16x4f32); the
+//               second and third take both operands as three bf16 pieces
+//               (tanh_layer_split). Only the per-world prologue (input noise)
+//               and epilogue (Gaussian sample, log-prob, PD targets) go
+//               through LDS, because each world's random stream is sequential
+//               and lives in one lane. Small launches give a tile of 16
+//               worlds to a workgroup of four waves instead (policy_team).
 #pragma once
 
 namespace phz {
@@ -205,8 +208,9 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 struct PolicyArgs {
   const f32x4* w1;     // [KU][NHB][64] x 4 fragments of W1 (host re-layout, zero padded)
-  const f32x4* w2;     // [NHB][NHB][64] x 4 fragments of W2, input block major
-  const f32x4* w3;     // [NHB][NOB][64] x 4 fragments of W3, input block major
+  const f32x4* w2;     // W2, input block major: [KB2][NHB][3][64] x 8 bf16 pieces (P::SPLIT), or
+                       // [NHB][NHB][64] x 4 floats
+  const f32x4* w3;     // W3 likewise, NOB output blocks
   const float* bias;   // b1[NHB*16] b2[NHB*16] b3[NOB*16], zero padded
   const float* stdv;   // [NO]
   float* obs;          // [NI][stride], this control step's history row (noised in place)
@@ -229,11 +233,15 @@ struct PolicyArgs {
 // angle. These 37 normals per world and control step are the part of the
 // policy kernel that does not overlap its MFMAs; the kernel fills the tables
 // at its start.
+__device__ __forceinline__ double uniform_of(u64 x) {
+  return fma((double)(unsigned)(x >> 32), 0x1p-32, (double)((unsigned)x >> 11) * 0x1p-53);
+}
+__device__ __forceinline__ double turns_of(u64 x) {
+  return fma((double)(unsigned)(x >> 32), 0x1p-26, (double)((unsigned)x >> 11) * 0x1p-47);
+}
 __device__ __forceinline__ void policy_uniforms(u64& s, double& u1, double& t) {
-  const u64 x1 = xorshift64(s);
-  const u64 x2 = xorshift64(s);
-  u1 = fma((double)(unsigned)(x1 >> 32), 0x1p-32, (double)((unsigned)x1 >> 11) * 0x1p-53);
-  t = fma((double)(unsigned)(x2 >> 32), 0x1p-26, (double)((unsigned)x2 >> 11) * 0x1p-47);
+  u1 = uniform_of(xorshift64(s));
+  t = turns_of(xorshift64(s));
 }
 __device__ __forceinline__ double policy_transform(double u1, double t) {
   const double k = rint(t);
@@ -343,12 +351,128 @@ __device__ __forceinline__ void mfma_layer(const f32x4* __restrict__ w, int lane
   }
 }
 
+// ── layers 2 and 3 in three bf16 pieces ──
+// An f32 is the exact sum of three bf16 values, each the rounding of what the
+// ones before it left (8 significant bits each, signed remainders):
+// x = h + m + l. A product then needs the six partial products of relative
+// size above 2^-24: hh, hm, mh, hl, lh, mm; the three dropped ones (ml, lm, ll)
+// are below 2^-26 of it. bf16 products are exact in f32 and the MFMA sums 32
+// of them with one rounding where the f32 MFMA rounds per 4, so the layer's
+// error against 64 bits is no larger than the f32 MFMA's (measured in
+// tests/test_gpu_policy_split.py). Six 16x16x32 bf16 MFMAs (16 cycles each)
+// replace eight 16x16x4 f32 ones (32 cycles each) per 32 inputs: 96 against
+// 256 cycles of matrix core, for 5.5 more VALU instructions per activation.
+// 29-256-256-8, us per launch (f32, split): 56, 41 at 4096 worlds, 122, 79 at
+// 65536, 241, 165 at 131072, there with the two-wave build's parked tiles and
+// priorities 161. What bounds the large launch now is VALU issue and MFMA
+// together: 8300 VALU instructions (the normals' f64, tanh, the split) and
+// 34000 cycles of MFMA per wave, which the two waves of a SIMD overlap by
+// little.
+// Taken where every weight of the two layers is zero or of magnitude in
+// [2^-100, 2^100] (the host checks on upload), so that no piece overflows or
+// is subnormal; their inputs are tanh values. The first layer stays f32: its
+// inputs are the caller's observations, of any range.
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef float f32x8 __attribute__((ext_vector_type(8)));
+
+struct Split3 { bf16x8 h, m, l; };
+__device__ __forceinline__ Split3 split3(f32x4 a, f32x4 b) {
+  const f32x8 x = __builtin_shufflevector(a, b, 0, 1, 2, 3, 4, 5, 6, 7);
+  Split3 s;
+  s.h = __builtin_convertvector(x, bf16x8);
+  const f32x8 r = x - __builtin_convertvector(s.h, f32x8);
+  s.m = __builtin_convertvector(r, bf16x8);
+  s.l = __builtin_convertvector(r - __builtin_convertvector(s.m, f32x8), bf16x8);
+  return s;
+}
+__device__ __forceinline__ f32x4 mfma32(bf16x8 a, bf16x8 b, f32x4 c) {
+  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
+}
+// acc[cb] += W B over one block of 32 inputs, the small partial products
+// first; the columns alternate, so consecutive MFMAs do not depend.
+template <int CB>
+__device__ __forceinline__ void mfma_split(const Split3& w, const Split3 (&b)[CB], f32x4 (&acc)[CB]) {
+#pragma unroll
+  for (int cb = 0; cb < CB; cb++) acc[cb] = mfma32(w.l, b[cb].h, acc[cb]);
+#pragma unroll
+  for (int cb = 0; cb < CB; cb++) acc[cb] = mfma32(w.h, b[cb].l, acc[cb]);
+#pragma unroll
+  for (int cb = 0; cb < CB; cb++) acc[cb] = mfma32(w.m, b[cb].m, acc[cb]);
+#pragma unroll
+  for (int cb = 0; cb < CB; cb++) acc[cb] = mfma32(w.m, b[cb].h, acc[cb]);
+#pragma unroll
+  for (int cb = 0; cb < CB; cb++) acc[cb] = mfma32(w.h, b[cb].m, acc[cb]);
+#pragma unroll
+  for (int cb = 0; cb < CB; cb++) acc[cb] = mfma32(w.h, b[cb].h, acc[cb]);
+}
+__device__ __forceinline__ Split3 weight_pieces(const f32x4* w, int t, int lane) {
+  const bf16x8* p = (const bf16x8*)w + (size_t)t * 192 + lane;
+  return Split3{p[0], p[64], p[128]};
+}
+
+// As mfma_layer, on tanh of the input tiles h, taken two at a time (32 inputs;
+// an odd last tile is paired with zeros). The weights are [kb2][ob] triples of
+// pieces, streamed in that order with PF triples in flight (4 to 6 measured
+// the same). PARK = 0: the tanh of the next pair of tiles is spread over this
+// pair's output blocks, where it issues while the MFMAs run. PARK > 0: every
+// tanh first, and the last PARK tiles wait for their turn in LDS (`park`), for
+// a wave that would have to spill them.
+template <int PARK, int NHB_, int NOB_, int CB>
+__device__ __forceinline__ void tanh_layer_split(const f32x4* __restrict__ w, int lane, f32x4 (&acc)[NOB_][CB],
+                                                 f32x4 (&h)[NHB_][CB], f32x4* park) {
+  constexpr int KB2 = (NHB_ + 1) / 2, NT = KB2 * NOB_;
+  constexpr int PF = NT < 3 ? NT : 3;
+  constexpr int KEEP = NHB_ - PARK;  // tiles that stay in registers
+  Split3 ring[PF];
+#pragma unroll
+  for (int t = 0; t < PF; t++) ring[t] = weight_pieces(w, t, lane);
+  const f32x4 zero = {0.0f, 0.0f, 0.0f, 0.0f};
+  // Value e of a pair of tiles: tile, column, register.
+  auto squash = [&](auto K, auto E) {
+    constexpr int e = decltype(E)::value, tile = 2 * decltype(K)::value + e / (4 * CB);
+    if constexpr (tile < NHB_) {
+      float& x = *((float*)&h[tile][(e / 4) % CB] + e % 4);
+      x = tanh_mlp(x);
+    }
+  };
+  sfor<0, (PARK > 0 ? KB2 : 1)>([&](auto K) { sfor<0, 8 * CB>([&](auto E) { squash(K, E); }); });
+  sfor<KEEP, NHB_>([&](auto I) {
+    constexpr int i = decltype(I)::value;
+#pragma unroll
+    for (int cb = 0; cb < CB; cb++) park[((i - KEEP) * CB + cb) * 64 + lane] = h[i][cb];
+  });
+  auto tile = [&](auto I, int cb) {
+    constexpr int i = decltype(I)::value;
+    if constexpr (i >= NHB_) return zero;
+    else if constexpr (i < KEEP) return h[i][cb];
+    else return park[((i - KEEP) * CB + cb) * 64 + lane];
+  };
+  sfor<0, KB2>([&](auto K) {
+    constexpr int kb = decltype(K)::value;
+    Split3 b[CB];
+#pragma unroll
+    for (int cb = 0; cb < CB; cb++) b[cb] = split3(tile(ic<2 * kb>{}, cb), tile(ic<2 * kb + 1>{}, cb));
+    sfor<0, NOB_>([&](auto O) {
+      constexpr int o = decltype(O)::value, t = kb * NOB_ + o;
+      const Split3 wa = ring[t % PF];
+      if constexpr (t + PF < NT) ring[t % PF] = weight_pieces(w, t + PF, lane);
+      mfma_split<CB>(wa, b, acc[o]);
+      if constexpr (PARK == 0 && kb + 1 < KB2)
+        sfor<8 * CB * o / NOB_, 8 * CB * (o + 1) / NOB_>([&](auto E) { squash(ic<kb + 1>{}, E); });
+      __builtin_amdgcn_sched_barrier(0);
+    });
+  });
+}
+
 // v_mfma_f32_16x16x4f32 lane layout: A[i][k] in lane i + 16 k, B[k][j] in
 // lane j + 16 k, D[i][j] in lane j + 16 (i / 4), register i % 4.
 // Layer l computes H_l^T = tanh(W_l H_{l-1}^T + b_l): rows are neurons, columns
 // worlds. For the next layer, k-step s of input block kb uses register s of
 // the previous output tile, i.e. lane j + 16 g supplies neuron 16 kb + 4 g + s
 // of world j; the host lays W out to match (phz_host.cpp, policy_fragments).
+// The bf16 16x16x32 takes 8 values per lane, k = 8 g + s in lane group g, of
+// both operands: components 0..3 are neurons 32 kb + 4 g + s, components 4..7
+// neurons 32 kb + 16 + 4 g + (s - 4), the two tiles of the pair.
 // Inputs with observation noise, the prologue's normals per world.
 template <class P> constexpr int noised_inputs() {
   int c = 0;
@@ -356,8 +480,53 @@ template <class P> constexpr int noised_inputs() {
   return c;
 }
 
+// One world's sample (policy_reference, policy_pipeline.rs:488-520): every
+// servo gets its base target, then each action k: AR(1) noise, sample,
+// log-prob, the clamped action onto its slot's base. normal(k) is action k's
+// normal; the calls come in order (products and sums are fused as written, so
+// that every form of the kernel rounds alike). base[j] is servo j's base target and z[k]
+// the AR(1) state before the step.
+template <class P, class T, class NF>
+__device__ __forceinline__ void policy_sample(const PolicyArgs& a, int my, const float* mean, const T (&base)[P::NPD],
+                                              const float (&z)[P::NO], NF normal) {
+  constexpr int NO = P::NO, NPD = P::NPD;
+  const int S = a.stride;
+  T* tgt = (T*)a.targets;
+#pragma unroll
+  for (int j = 0; j < NPD; j++) tgt[(size_t)j * S + my] = base[j];
+  const float rho = float(P::rho);
+  const float keep = sqrtf(fmaxf(0.0f, 1.0f - rho * rho));
+  const float half_ln_2pi = 0.91893853320467274178f;
+  float logp = 0.0f;
+#pragma unroll
+  for (int k = 0; k < NO; k++) {
+    const float mk = mean[k];
+    const float zk = fmaf(rho, z[k], keep * normal(k));
+    a.z[(size_t)k * S + my] = zk;
+    const float sd = a.stdv[k];
+    const float act = fmaf(sd, zk, mk);
+    const float zi = (act - mk) / sd;
+    logp += fmaf(-0.5f * zi, zi, -logf(sd)) - half_ln_2pi;
+    a.out[(size_t)k * S + my] = act;
+    const float lim = float(P::clamp[k]);
+    // clamp(-lim, lim) that passes NaN through, as f64::clamp does.
+    const float applied = act < -lim ? -lim : (act > lim ? lim : act);
+    const int slot = P::slot[k];
+    tgt[(size_t)slot * S + my] = base[slot] + T(applied);
+  }
+  a.out[(size_t)NO * S + my] = logp;
+}
+
+template <class P, class T>
+__device__ __forceinline__ void sample_state(const PolicyArgs& a, int my, T (&base)[P::NPD], float (&z)[P::NO]) {
+#pragma unroll
+  for (int j = 0; j < P::NPD; j++) base[j] = ((const T*)a.base)[(size_t)j * a.stride + my];
+#pragma unroll
+  for (int k = 0; k < P::NO; k++) z[k] = a.z[(size_t)k * a.stride + my];
+}
+
 template <class P, class T> __device__ __forceinline__ void policy_wave(const PolicyArgs& a, float* lds) {
-  constexpr int NI = P::NI, NO = P::NO, CB = P::CB, NHB = P::NHB, NOB = P::NOB, KU = P::KU, NPD = P::NPD;
+  constexpr int NI = P::NI, NO = P::NO, CB = P::CB, NHB = P::NHB, NOB = P::NOB, KU = P::KU;
   constexpr int WPW = 16 * CB;     // worlds per wave
   constexpr int XS = 16 * KU + 1;  // LDS row stride of the input tile (floats)
   constexpr int MS = 16 * NOB + 1; // LDS row stride of the output tile
@@ -367,6 +536,13 @@ template <class P, class T> __device__ __forceinline__ void policy_wave(const Po
   const int my = w0 + lane;
   const bool own = lane < WPW && my < a.nworld;
   u64 rs = 0;
+  // Two-wave builds: the second wave of a SIMD issues first where both can, so
+  // that the two leave lockstep and one's VALU phases fall into the other's
+  // MFMAs (workgroups fill a SIMD's first wave, then its second; the order is
+  // no more than a hint): 149 -> 145 us at 131072 worlds.
+  if constexpr (P::PARK > 0) {
+    if ((blockIdx.x >> 10) & 1) __builtin_amdgcn_s_setprio(3);
+  }
 
   // Prologue: world w0 + lane reads its observation row, adds input noise in
   // index order (the noised value is what the history keeps), stages x in LDS.
@@ -385,7 +561,7 @@ template <class P, class T> __device__ __forceinline__ void policy_wave(const Po
 #pragma unroll
       for (int i = 0; i < NI; i++)
         if (P::noise[i] != 0.0) {
-          x[i] += float(P::noise[i]) * (float)nz[c++];
+          x[i] = fmaf(float(P::noise[i]), (float)nz[c++], x[i]);
           if (own) a.obs[(size_t)i * S + my] = x[i];
         }
     }
@@ -401,7 +577,7 @@ template <class P, class T> __device__ __forceinline__ void policy_wave(const Po
       if (i < NI && own) {
         x = a.obs[(size_t)i * S + my];
         if (P::noise[i] != 0.0) {
-          x += float(P::noise[i]) * (float)policy_normal(rs);
+          x = fmaf(float(P::noise[i]), (float)policy_normal(rs), x);
           a.obs[(size_t)i * S + my] = x;
         }
       }
@@ -416,16 +592,25 @@ template <class P, class T> __device__ __forceinline__ void policy_wave(const Po
   f32x4 h[NHB][CB];
   bias_tiles<NHB, CB>(a.bias, g, h);
   mfma_layer<KU, NHB, CB>(a.w1, lane, h, [&](int kb, int s, int cb) { return lds[(cb * 16 + r) * XS + 16 * kb + 4 * s + g]; });
-  tanh_tiles<NHB, CB>(h);
   // Layer 2: B = layer 1's output tiles, straight from registers.
   f32x4 h2[NHB][CB];
   bias_tiles<NHB, CB>(a.bias + 16 * NHB, g, h2);
-  mfma_layer<NHB, NHB, CB>(a.w2, lane, h2, [&](int kb, int s, int cb) { return h[kb][cb][s]; });
-  tanh_tiles<NHB, CB>(h2);
+  if constexpr (P::SPLIT) {
+    __syncthreads();  // the input tile's LDS is the parked tiles' now
+    tanh_layer_split<P::PARK, NHB, NHB, CB>(a.w2, lane, h2, h, (f32x4*)lds);
+  } else {
+    tanh_tiles<NHB, CB>(h);
+    mfma_layer<NHB, NHB, CB>(a.w2, lane, h2, [&](int kb, int s, int cb) { return h[kb][cb][s]; });
+  }
   // Layer 3: the action means.
   f32x4 m[NOB][CB];
   bias_tiles<NOB, CB>(a.bias + 32 * NHB, g, m);
-  mfma_layer<NHB, NOB, CB>(a.w3, lane, m, [&](int kb, int s, int cb) { return h2[kb][cb][s]; });
+  if constexpr (P::SPLIT) {
+    tanh_layer_split<0, NHB, NOB, CB>(a.w3, lane, m, h2, nullptr);
+  } else {
+    tanh_tiles<NHB, CB>(h2);
+    mfma_layer<NHB, NOB, CB>(a.w3, lane, m, [&](int kb, int s, int cb) { return h2[kb][cb][s]; });
+  }
   // Means to LDS, world-major, for the per-world epilogue.
   __syncthreads();
 #pragma unroll
@@ -436,40 +621,207 @@ template <class P, class T> __device__ __forceinline__ void policy_wave(const Po
       for (int j = 0; j < 4; j++) lds[(cb * 16 + r) * MS + ob * 16 + 4 * g + j] = m[ob][cb][j];
   __syncthreads();
 
-  // Epilogue (policy_reference, policy_pipeline.rs:488-520): every servo gets
-  // its base target, then each action k: AR(1) noise, sample, log-prob, the
-  // clamped action onto its slot's base. With half the lanes owning a world
-  // the actions' normals are drawn first, paired across the halves.
+  // With half the lanes owning a world the actions' normals are drawn first,
+  // paired across the halves.
   double na[NO];
   if constexpr (WPW == 32) policy_normals_paired<NO>(rs, lane, na);
   if (own) {
-    const T* base = (const T*)a.base;
-    T* tgt = (T*)a.targets;
-#pragma unroll
-    for (int j = 0; j < NPD; j++) tgt[(size_t)j * S + my] = base[(size_t)j * S + my];
-    const float rho = float(P::rho);
-    const float keep = sqrtf(fmaxf(0.0f, 1.0f - rho * rho));
-    const float half_ln_2pi = 0.91893853320467274178f;
-    float logp = 0.0f;
-#pragma unroll
-    for (int k = 0; k < NO; k++) {
-      const float mk = lds[lane * MS + k];
-      const float zk = rho * a.z[(size_t)k * S + my] + keep * (float)(WPW == 32 ? na[k] : policy_normal(rs));
-      a.z[(size_t)k * S + my] = zk;
-      const float sd = a.stdv[k];
-      const float act = mk + sd * zk;
-      const float zi = (act - mk) / sd;
-      logp += -0.5f * zi * zi - logf(sd) - half_ln_2pi;
-      a.out[(size_t)k * S + my] = act;
-      const float lim = float(P::clamp[k]);
-      // clamp(-lim, lim) that passes NaN through, as f64::clamp does.
-      const float applied = act < -lim ? -lim : (act > lim ? lim : act);
-      const int slot = P::slot[k];
-      tgt[(size_t)slot * S + my] = base[(size_t)slot * S + my] + T(applied);
-    }
-    a.out[(size_t)NO * S + my] = logp;
+    T base[P::NPD];
+    float z[NO];
+    sample_state<P, T>(a, my, base, z);
+    policy_sample<P, T>(a, my, lds + lane * MS, base, z, [&](int k) { return (float)(WPW == 32 ? na[k] : policy_normal(rs)); });
     a.rng[my] = rs;
   }
+}
+
+// ── small launches: a tile of 16 CB worlds to a workgroup of TW waves ──
+// One wave per tile leaves most SIMDs idle when a launch has few tiles, and
+// the launch then lasts as long as one wave's stream (29-256-256-8: 40 us at
+// 64 worlds, 44 at 16384; here 16 and 39). Here wave k computes the hidden neurons of blocks
+// k * BPW .. of both hidden layers for the whole tile, and passes them to the
+// others through LDS, already split into bf16 pieces and laid out as B
+// fragments. The streams' raw draws are one lane's work per world, the
+// Box-Muller transforms are spread over every lane. Every sum runs in
+// policy_wave's order: the two give the same bits.
+//
+// LDS: the draws (8 bytes each, later the hidden pieces: KB2 x 3 x CB x 1 KB),
+// the input tile [world][XS], the means [world][MS] and the actions' normals.
+template <class P> constexpr int team_draws() { return 2 * (noised_inputs<P>() + P::NO) * 16 * P::CB * 8; }
+template <class P> constexpr int team_pieces() { return ((P::NHB + 1) / 2) * 3 * P::CB * 1024; }
+template <class P> constexpr int team_front() {
+  return team_draws<P>() > team_pieces<P>() ? team_draws<P>() : team_pieces<P>();
+}
+template <class P> constexpr int team_lds_bytes() {
+  return team_front<P>() + 16 * P::CB * (16 * P::KU + 1 + 16 * P::NOB + 1 + P::NO) * 4;
+}
+
+// h[j] is tile blk0 + j: its pieces into the halves of fragment (blk / 2).
+template <int CB, int BPW>
+__device__ __forceinline__ void put_pieces(bf16x8* pieces, const f32x4 (&h)[BPW][CB], int blk0, int nhb, int lane) {
+#pragma unroll
+  for (int j = 0; j < BPW; j += 2) {
+    const int blk = blk0 + j;
+    if (blk >= nhb) continue;
+    const f32x4 zero = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int cb = 0; cb < CB; cb++) {
+      const Split3 s = split3(h[j][cb], blk + 1 < nhb ? h[j + 1][cb] : zero);
+      bf16x8* p = pieces + ((size_t)(blk / 2) * 3 * CB + cb) * 64 + lane;
+      p[0] = s.h;
+      p[CB * 64] = s.m;
+      p[2 * CB * 64] = s.l;
+    }
+  }
+}
+template <int CB> __device__ __forceinline__ void get_pieces(const bf16x8* pieces, int kb, int lane, Split3 (&b)[CB]) {
+#pragma unroll
+  for (int cb = 0; cb < CB; cb++) {
+    const bf16x8* p = pieces + ((size_t)kb * 3 * CB + cb) * 64 + lane;
+    b[cb] = Split3{p[0], p[CB * 64], p[2 * CB * 64]};
+  }
+}
+
+template <class P, class T> __device__ __forceinline__ void policy_team(const PolicyArgs& a, char* lds) {
+  constexpr int NI = P::NI, NO = P::NO, CB = P::CB, NHB = P::NHB, NOB = P::NOB, KU = P::KU, TW = P::TW;
+  constexpr int W = 16 * CB, XS = 16 * KU + 1, MS = 16 * NOB + 1, KB2 = (NHB + 1) / 2;
+  constexpr int BPW = 2 * ((KB2 + TW - 1) / TW);  // hidden blocks per wave, whole pairs
+  constexpr int NN = noised_inputs<P>(), ND = NN + NO;
+  u64* draws = (u64*)lds;                          // [ND][2][W]
+  bf16x8* pieces = (bf16x8*)lds;                   // [KB2][3][CB][64]
+  float* x = (float*)(lds + team_front<P>());      // [W][XS]
+  float* mean = x + W * XS;                        // [W][MS]
+  float* nact = mean + W * MS;                     // [NO][W]
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int w0 = blockIdx.x * W, S = a.stride;
+
+  // What later phases read from memory is loaded ahead of the barriers before
+  // them: layer 1's weights (of a narrow input) and the sample's state here,
+  // layer 2's first weights before layer 1, layer 3's before its inputs are
+  // exchanged.
+  constexpr bool PRE = KU <= 2;
+  f32x4 w1f[BPW][PRE ? KU : 1];
+  const int blk0 = wave * BPW;
+  auto block = [&](int j) { return blk0 + j < NHB ? blk0 + j : NHB - 1; };
+  if constexpr (PRE) {
+#pragma unroll
+    for (int j = 0; j < BPW; j++)
+#pragma unroll
+      for (int kb = 0; kb < KU; kb++) w1f[j][kb] = a.w1[(kb * NHB + block(j)) * 64 + lane];
+  }
+  const bool sampler = tid < W && w0 + tid < a.nworld;
+  T base[P::NPD];
+  float z[NO];
+  if (sampler) sample_state<P, T>(a, w0 + tid, base, z);
+
+  // Raw draws in stream order (inputs, then actions) by one lane per world of
+  // the first wave; the other waves stage the observation rows.
+  if (tid < W) {
+    const int my = w0 + tid;
+    u64 rs = my < a.nworld ? a.rng[my] : 1;
+#pragma unroll 4
+    for (int d = 0; d < 2 * ND; d++) draws[d * W + tid] = xorshift64(rs);
+    if (my < a.nworld) a.rng[my] = rs;
+  }
+  for (int e = tid; e < 16 * KU * W; e += 64 * TW) {
+    const int i = e / W, w = e % W;
+    x[w * XS + i] = i < NI && w0 + w < a.nworld ? a.obs[(size_t)i * S + w0 + w] : 0.0f;
+  }
+  __syncthreads();
+  for (int e = tid; e < ND * W; e += 64 * TW) {
+    const int d = e / W, w = e % W;
+    const u64 x1 = draws[(2 * d) * W + w], x2 = draws[(2 * d + 1) * W + w];
+    const float n = (float)policy_transform(uniform_of(x1), turns_of(x2));
+    if (d < NN) {
+      const int i = P::noised[d];
+      const float xi = fmaf(P::scale[d], n, x[w * XS + i]);
+      x[w * XS + i] = xi;
+      if (w0 + w < a.nworld) a.obs[(size_t)i * S + w0 + w] = xi;
+    } else {
+      nact[(d - NN) * W + w] = n;
+    }
+  }
+  __syncthreads();
+
+  const int r = lane & 15, g = lane >> 4;
+  auto w2_at = [&](int kb, int j) { return weight_pieces(a.w2, kb * NHB + block(j), lane); };
+  Split3 wn[BPW];
+#pragma unroll
+  for (int j = 0; j < BPW; j++) wn[j] = w2_at(0, j);
+  // Layer 1, this wave's blocks (one past the last block repeats it and is
+  // not stored).
+  f32x4 h[BPW][CB];
+#pragma unroll
+  for (int j = 0; j < BPW; j++) {
+    f32x4 acc[1][CB];
+    bias_tiles<1, CB>(a.bias + 16 * block(j), g, acc);
+#pragma unroll
+    for (int kb = 0; kb < KU; kb++) {
+      f32x4 wa;
+      if constexpr (PRE) wa = w1f[j][kb];
+      else wa = a.w1[(kb * NHB + block(j)) * 64 + lane];
+#pragma unroll
+      for (int s = 0; s < 4; s++)
+#pragma unroll
+        for (int cb = 0; cb < CB; cb++) acc[0][cb] = mfma4(wa[s], x[(cb * 16 + r) * XS + 16 * kb + 4 * s + g], acc[0][cb]);
+    }
+#pragma unroll
+    for (int cb = 0; cb < CB; cb++) h[j][cb] = acc[0][cb];
+  }
+  tanh_tiles<BPW, CB>(h);
+  put_pieces<CB, BPW>(pieces, h, blk0, NHB, lane);
+  __syncthreads();
+  // Layer 2: every input pair, this wave's output blocks; the next pair's
+  // weights load while this one multiplies.
+  f32x4 h2[BPW][CB];
+#pragma unroll
+  for (int j = 0; j < BPW; j++) {
+    f32x4 acc[1][CB];
+    bias_tiles<1, CB>(a.bias + 16 * NHB + 16 * block(j), g, acc);
+#pragma unroll
+    for (int cb = 0; cb < CB; cb++) h2[j][cb] = acc[0][cb];
+  }
+#pragma unroll
+  for (int kb = 0; kb < KB2; kb++) {
+    Split3 b[CB];
+    get_pieces<CB>(pieces, kb, lane, b);
+#pragma unroll
+    for (int j = 0; j < BPW; j++) {
+      const Split3 wa = wn[j];
+      if (kb + 1 < KB2) wn[j] = w2_at(kb + 1, j);
+      mfma_split<CB>(wa, b, h2[j]);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  }
+  constexpr int P3 = KB2 < 3 ? KB2 : 3;  // layer 3's weights in flight
+  Split3 w3[P3];
+  if (wave < NOB) {
+#pragma unroll
+    for (int kb = 0; kb < P3; kb++) w3[kb] = weight_pieces(a.w3, kb * NOB + wave, lane);
+  }
+  tanh_tiles<BPW, CB>(h2);
+  __syncthreads();  // every wave is past its reads of layer 1's pieces
+  put_pieces<CB, BPW>(pieces, h2, blk0, NHB, lane);
+  __syncthreads();
+  // Layer 3: output block k on wave k.
+  if (wave < NOB) {
+    f32x4 acc[1][CB];
+    bias_tiles<1, CB>(a.bias + 32 * NHB + 16 * wave, g, acc);
+#pragma unroll
+    for (int kb = 0; kb < KB2; kb++) {
+      const Split3 wa = w3[kb % P3];
+      if (kb + P3 < KB2) w3[kb % P3] = weight_pieces(a.w3, (kb + P3) * NOB + wave, lane);
+      Split3 b[CB];
+      get_pieces<CB>(pieces, kb, lane, b);
+      mfma_split<CB>(wa, b, acc[0]);
+    }
+#pragma unroll
+    for (int cb = 0; cb < CB; cb++)
+#pragma unroll
+      for (int j = 0; j < 4; j++) mean[(cb * 16 + r) * MS + wave * 16 + 4 * g + j] = acc[0][cb][j];
+  }
+  __syncthreads();
+  if (sampler)
+    policy_sample<P, T>(a, w0 + tid, mean + tid * MS, base, z, [&](int k) { return nact[k * W + tid]; });
 }
 
 }  // namespace phz

@@ -1076,7 +1076,11 @@ struct PolicyD {
   std::vector<double> clamp;  // n_out (the scalar broadcast when no per-slot clamp, PolicySpec::clamp_row)
   std::vector<int> slots;     // n_out
   double rho = 0;
+  // Layers 2 and 3 as bf16 pieces (tanh_layer_split in phz_control.h): the
+  // kernels' form for weights it represents, else f32 (set_policy_weights).
+  bool split = true;
   int nhb() const { return (hidden + 15) / 16; }
+  int kb2() const { return (nhb() + 1) / 2; }
   int nob() const { return (n_out + 15) / 16; }
   int ku() const { return (n_in + 15) / 16; }  // 16-input groups of layer 1
   // Worlds per wave = 16 * cb: as many 16-world column blocks as keep both
@@ -1088,15 +1092,50 @@ struct PolicyD {
   }
   // Fragment buffer (floats): W1 [ku][nhb][64][4], W2 [nhb][nhb][64][4],
   // W3 [nhb][nob][64][4] (input block major, the order the kernel streams
-  // them), then the biases.
+  // them), then the biases. Split: W2 [kb2][nhb][3][64] x 8 bf16 (4 floats),
+  // W3 [kb2][nob][3][64] x 8 bf16, the larger of the two layouts.
+  size_t in_blocks() const { return split ? 3 * (size_t)kb2() : (size_t)nhb(); }
   size_t off_w2() const { return (size_t)ku() * nhb() * 256; }
-  size_t off_w3() const { return off_w2() + (size_t)nhb() * nhb() * 256; }
-  size_t off_bias() const { return off_w3() + (size_t)nhb() * nob() * 256; }
+  size_t off_w3() const { return off_w2() + in_blocks() * nhb() * 256; }
+  size_t off_bias() const { return off_w3() + in_blocks() * nob() * 256; }
   size_t frag_floats() const { return off_bias() + 16 * (size_t)(2 * nhb() + nob()); }
   bool same_shape(const PolicyD& o) const {
     return n_in == o.n_in && hidden == o.hidden && n_out == o.n_out && history == o.history;
   }
 };
+
+// The bf16 nearest x (ties to even), as its 16 bits; x finite.
+uint16_t bf16_bits(float x) {
+  uint32_t u;
+  std::memcpy(&u, &x, 4);
+  return (uint16_t)((u + 0x7fffu + ((u >> 16) & 1u)) >> 16);
+}
+float bf16_value(uint16_t b) {
+  const uint32_t u = (uint32_t)b << 16;
+  float x;
+  std::memcpy(&x, &u, 4);
+  return x;
+}
+
+// Whether the policy kernels run layers 2 and 3 in bf16 pieces: three of them
+// hold every weight with no piece infinite or subnormal (zero, or a magnitude
+// in [2^-100, 2^100]), and a layer has at least 32 inputs, from where its
+// error against 64 bits is below the f32 MFMA's (ratio of the two over weight
+// scales 0.05 to 3: 0.73-0.96 at widths 32 to 256, 0.77-1.03 at 24, 0.79-1.18
+// at 16, where nothing is gained in time either: 20.0 against 20.1 us).
+constexpr int kSplitMinHidden = 32;
+bool policy_splits(const PolicyD& p, const double* w) {
+  if (p.hidden < kSplitMinHidden) return false;
+  const size_t h = p.hidden, b2 = h * p.n_in + h, b3 = b2 + h * h + h;
+  auto fits = [&](size_t from, size_t n) {
+    for (size_t k = from; k < from + n; k++) {
+      const float x = std::fabs((float)w[k]);
+      if (!(x == 0.0f || (x >= 0x1p-100f && x <= 0x1p100f))) return false;
+    }
+    return true;
+  };
+  return fits(b2, h * h) && fits(b3, h * p.n_out);
+}
 
 // The MLP weights in the policy kernel's MFMA fragment order (see
 // policy_wave in phz_control.h). Input order is the reference's flat
@@ -1118,15 +1157,35 @@ void policy_fragments(const PolicyD& p, const double* w, std::vector<float>& out
           const int n = hb * 16 + (l & 15), i = 16 * u + 4 * s + (l >> 4);
           if (n < NH && i < NI) out[(((size_t)u * NHB + hb) * 64 + l) * 4 + s] = (float)W1[(size_t)n * NI + i];
         }
+  // Split layers 2 and 3: component s of piece q of fragment (kb, ob), lane l =
+  // piece q of W[16 ob + l%16][32 kb + 4 (l/16) + s (+ 12 from s = 4 on)].
+  auto pieces = [&](const double* W, int rows, int obs, size_t off) {
+    for (int kb = 0; kb < p.kb2(); kb++)
+      for (int ob = 0; ob < obs; ob++)
+        for (int l = 0; l < 64; l++)
+          for (int s = 0; s < 8; s++) {
+            const int o = ob * 16 + (l & 15), i = 32 * kb + 4 * (l >> 4) + (s < 4 ? s : s + 12);
+            float rest = o < rows && i < NH ? (float)W[(size_t)o * NH + i] : 0.0f;
+            for (int q = 0; q < 3; q++) {
+              const uint16_t b = bf16_bits(rest);
+              std::memcpy((char*)&out[off] + ((((size_t)kb * obs + ob) * 3 + q) * 64 + l) * 16 + 2 * s, &b, 2);
+              rest -= bf16_value(b);
+            }
+          }
+  };
+  if (p.split) {
+    pieces(W2, NH, NHB, p.off_w2());
+    pieces(W3, NO, NOB, p.off_w3());
+  }
   // Layers 2 and 3: component s of fragment (kb, ob), lane l = W[16 ob + l%16][16 kb + 4 (l/16) + s].
-  for (int kb = 0; kb < NHB; kb++)
+  for (int kb = 0; kb < NHB && !p.split; kb++)
     for (int hb = 0; hb < NHB; hb++)
       for (int l = 0; l < 64; l++)
         for (int s = 0; s < 4; s++) {
           const int n2 = hb * 16 + (l & 15), n1 = kb * 16 + 4 * (l >> 4) + s;
           if (n2 < NH && n1 < NH) out[p.off_w2() + (((size_t)kb * NHB + hb) * 64 + l) * 4 + s] = (float)W2[(size_t)n2 * NH + n1];
         }
-  for (int kb = 0; kb < NHB; kb++)
+  for (int kb = 0; kb < NHB && !p.split; kb++)
     for (int ob = 0; ob < NOB; ob++)
       for (int l = 0; l < 64; l++)
         for (int s = 0; s < 4; s++) {
@@ -1237,27 +1296,49 @@ std::string gen_obs_source(const ModelD& m, const PolicyD* p, bool f64) {
 }
 
 // Policy kernel: widths, action wiring and noise scales compiled in.
-// two_waves: as gen_source's, two resident waves per SIMD.
-std::string gen_policy_source(const PolicyD& p, int npd, bool f64, bool two_waves = false) {
+// two_waves: as gen_source's, two resident waves per SIMD. team: a workgroup
+// of kTeamWaves waves per 16 worlds (policy_team).
+constexpr int kTeamWaves = 4;
+std::string gen_policy_source(const PolicyD& p, int npd, bool f64, bool two_waves = false, bool team = false) {
   const std::string T = f64 ? "double" : "float";
   std::string s = kDeviceSrc;
   s += "\n";
   s += kControlSrc;
-  const int cb = p.cb();
-  const int lds = 16 * cb * std::max(16 * p.ku() + 1, 16 * p.nob() + 1);
+  const int cb = team ? 1 : p.cb();
+  // Two-wave builds park tiles of layer 1 in LDS, up to 16 KB per wave (8
+  // waves of 18 KB a CU) instead of spilling them: at hidden 256, 284 -> 52 B
+  // of scratch per lane, 155 -> 149 us.
+  const int park = two_waves && p.split ? std::min(16 / cb, p.nhb() - 2) : 0;
+  const int lds = std::max(16 * cb * std::max(16 * p.ku() + 1, 16 * p.nob() + 1), park * cb * 256);
   std::ostringstream o;
   o << "\n// ---- policy shape ----\nstruct Pol {\n";
   o << "  static constexpr int NI = " << p.n_in << ", NH = " << p.hidden << ", NO = " << p.n_out << ", NHB = " << p.nhb()
-    << ", NOB = " << p.nob() << ", KU = " << p.ku() << ", CB = " << cb << ", NPD = " << npd << ", LDS = " << lds << ";\n";
+    << ", NOB = " << p.nob() << ", KU = " << p.ku() << ", CB = " << cb << ", NPD = " << npd << ", LDS = " << lds
+    << ", TW = " << kTeamWaves << ", PARK = " << park << ";\n";
+  o << "  static constexpr bool SPLIT = " << (p.split ? "true" : "false") << ";\n";
+  std::vector<int> noised;  // the inputs with noise, in order
+  for (int k = 0; k < p.n_in; k++) if (p.noise[k] != 0.0) noised.push_back(k);
+  const int nn = std::max<int>((int)noised.size(), 1);
+  auto at = [&](int k) { return k < (int)noised.size() ? noised[k] : 0; };
+  o << "  static constexpr int noised[" << nn << "] = " << arr1(nn, [&](int k) { return std::to_string(at(k)); }) << ";\n";
+  o << "  static constexpr float scale[" << nn << "] = "
+    << arr1(nn, [&](int k) { return "float(" + num(p.noise[at(k)]) + ")"; }) << ";\n";
   o << "  static constexpr double rho = " << num(p.rho) << ";\n";
   o << "  static constexpr double noise[" << p.n_in << "] = " << arr1(p.n_in, [&](int k) { return num(p.noise[k]); }) << ";\n";
   o << "  static constexpr double clamp[" << p.n_out << "] = " << arr1(p.n_out, [&](int k) { return num(p.clamp[k]); }) << ";\n";
   o << "  static constexpr int slot[" << p.n_out << "] = " << arr1(p.n_out, [&](int k) { return std::to_string(p.slots[k]); })
     << ";\n};\n";
   s += o.str();
+  if (team) {
+    s += "extern \"C\" __global__ void __launch_bounds__(" + std::to_string(64 * kTeamWaves) + ") phz_policy(phz::PolicyArgs a) {\n";
+    s += "  __shared__ __align__(16) char lds[phz::team_lds_bytes<Pol>()];\n";
+    s += "  if (threadIdx.x < 64) phz::fill_tables(threadIdx.x);\n  __syncthreads();\n";
+    s += "  phz::policy_team<Pol, " + T + ">(a, lds);\n}\n";
+    return s;
+  }
   s += std::string("extern \"C\" __global__ void __launch_bounds__(64)") +
        (two_waves ? " __attribute__((amdgpu_waves_per_eu(2, 2)))" : "") + " phz_policy(phz::PolicyArgs a) {\n";
-  s += "  __shared__ float lds[Pol::LDS];\n";
+  s += "  __shared__ __align__(16) float lds[Pol::LDS];\n";
   s += "  phz::fill_tables(threadIdx.x);\n  __syncthreads();\n";  // the normals' f64 log, sine and cosine tables
   s += "  phz::policy_wave<Pol, " + T + ">(a, lds);\n}\n";
   return s;
@@ -1349,6 +1430,7 @@ struct phz_sim {
   uint64_t ctl_epoch = 1;       // bumped when the model, PD table or policy spec changes
   bool policy_on = false;
   PolicyD pol;
+  bool pol_team = false;        // pol_k is the workgroup-per-tile form
   float* pw = nullptr;          // weight fragments and biases
   float* pstd = nullptr;        // [n_out]
   float* obs_hist = nullptr;    // [history][n_in][stride]
@@ -1587,6 +1669,17 @@ struct phz_sim {
   float* obs_row(uint32_t step) const { return obs_hist + (size_t)step * pol.n_in * stride; }
   float* out_row(uint32_t step) const { return out_hist + (size_t)step * (pol.n_out + 1) * stride; }
 
+  // Whether a policy launch of this size runs the workgroup-per-tile kernel:
+  // up to four 16-world tiles per CU. us per launch, one wave per tile against
+  // it (29 inputs, 8 actions): hidden 256, 64 worlds 40 / 16, 4096 41 / 18,
+  // 8192 42 / 23, 16384 44 / 39, 24576 46 / 51; hidden 64, 4096 26 / 13, 16384
+  // 27 / 18, 24576 28 / 25, 65536 31 / 49. PHZ_POLICY_TEAM=0|1 forces it off or
+  // on (tests, tuning).
+  bool team_pays() const {
+    if (!pol.split) return false;
+    if (const char* e = std::getenv("PHZ_POLICY_TEAM")) return e[0] == '1';
+    return ((long)nworld + 15) / 16 <= 4L * std::max(feat.cus, 1);
+  }
   // Compile (and with `load`, load) the FK/observation or the policy kernel
   // for the current configuration epoch.
   bool ensure_ctl(bool policy_kernel, bool load) {
@@ -1597,7 +1690,8 @@ struct phz_sim {
       k.reset();
     }
     if (!k.code) {
-      const std::string src = policy_kernel ? gen_policy_source(pol, feat.npd, f64)
+      if (policy_kernel) pol_team = team_pays();
+      const std::string src = policy_kernel ? gen_policy_source(pol, feat.npd, f64, false, pol_team)
                                             : gen_obs_source(model, policy_on ? &pol : nullptr, f64);
       std::string e;
       k.code = compile_source(src, Build::Finite, e);
@@ -1608,12 +1702,13 @@ struct phz_sim {
       // two resident waves per SIMD (the same build: the same bits) overlaps
       // one wave's VALU work with another's MFMAs: on the ant control workload
       // (131072 worlds, 4096 waves) 0.255 -> 0.224 ms per launch with 164 B
-      // of spills per lane, rollout 16.99 -> 15.35 ms. Taken while it spills
+      // of spills per lane, rollout 16.99 -> 15.35 ms (all in f32; the split
+      // layers' figures are with tanh_layer_split). Taken while it spills
       // at most 512 B per lane; PHZ_TWO_WAVES=0 keeps one wave per SIMD.
       const char* tw = std::getenv("PHZ_TWO_WAVES");
       const long waves = ((long)nworld + 16L * pol.cb() - 1) / (16L * pol.cb());
       const int64_t regs = remark_value(k.code->log, "VGPRs:") + std::max<int64_t>(remark_value(k.code->log, "AGPRs:"), 0);
-      if (policy_kernel && !(tw && tw[0] == '0') && regs > 256 && waves > 4L * std::max(feat.cus, 1)) {
+      if (policy_kernel && !pol_team && !(tw && tw[0] == '0') && regs > 256 && waves > 4L * std::max(feat.cus, 1)) {
         std::string e2;
         auto c2 = compile_source(gen_policy_source(pol, feat.npd, f64, true), Build::Finite, e2);
         const int64_t sc = c2 ? remark_value(c2->log, "ScratchSize [bytes/lane]:") : -1;
@@ -1640,12 +1735,12 @@ struct phz_sim {
     return hip_ok(hipModuleLaunchKernel(obs_k.fn, grid, 1, 1, 64, 1, 1, 0, stream, params, nullptr), "obs kernel launch");
   }
   bool launch_policy(uint32_t step) {
-    const int wpw = 16 * pol.cb();
+    const int wpw = pol_team ? 16 : 16 * pol.cb();
     PolicyArgs a{pw, pw + pol.off_w2(), pw + pol.off_w3(), pw + pol.off_bias(), pstd, obs_row(step), out_row(step),
                  prng, pz, pbase, targets, nworld, stride};
     void* params[] = {&a};
     const unsigned grid = (unsigned)((nworld + wpw - 1) / wpw);
-    return hip_ok(hipModuleLaunchKernel(pol_k.fn, grid, 1, 1, 64, 1, 1, 0, stream, params, nullptr),
+    return hip_ok(hipModuleLaunchKernel(pol_k.fn, grid, 1, 1, pol_team ? 64 * kTeamWaves : 64, 1, 1, 0, stream, params, nullptr),
                   "policy kernel launch");
   }
   // Everything run_policy needs, checked on the host (mod.rs:1209-1231).
@@ -2480,6 +2575,7 @@ int phz_enable_policy(phz_sim* s, const double* ops, uint32_t n_in, const double
   if (phz_enable_kinematics(s)) return 1;
   if (!set_device(s)) return 1;
   const bool reuse = s->policy_on && s->pol.same_shape(p);
+  p.split = reuse ? s->pol.split : p.hidden >= kSplitMinHidden;  // kept weights stay in their layout
   if (s->stream) hipStreamSynchronize(s->stream);
   if (s->rexec) { hipGraphExecDestroy(s->rexec); s->rexec = nullptr; }
   s->pol = p;
@@ -2513,6 +2609,11 @@ int phz_set_policy_weights(phz_sim* s, const double* weights, uint64_t n) {
   if (!weights) return s->fail("null weights");
   if (!s->has_device()) return s->fail("host-only sim has no device buffers");
   if (!set_device(s)) return 1;
+  const bool split = policy_splits(s->pol, weights);
+  if (split != s->pol.split) {  // the other layout's kernel; frees nothing (pw holds the larger layout)
+    s->pol.split = split;
+    s->ctl_epoch++;
+  }
   std::vector<float> frag;
   policy_fragments(s->pol, weights, frag);
   if (!s->hip_ok(hipMemcpyAsync(s->pw, frag.data(), frag.size() * 4, hipMemcpyHostToDevice, s->stream), "upload weights"))
@@ -2681,8 +2782,9 @@ int phz_control_kernel_info(phz_sim* s, int which, int64_t* info) {
   info[1] = remark_value(log, "AGPRs:");
   info[2] = remark_value(log, "SGPRs:");
   info[3] = remark_value(log, "ScratchSize [bytes/lane]:");
-  info[4] = 64;
-  info[5] = which == 1 ? 16 * s->pol.cb() : 64;
+  const bool team = which == 1 && s->pol_team;
+  info[4] = team ? 64 * kTeamWaves : 64;
+  info[5] = team ? 16 : which == 1 ? 16 * s->pol.cb() : 64;
   return 0;
 }
 

@@ -1,0 +1,93 @@
+"""The policy kernel's layers 2 and 3 in bf16 pieces, and its workgroup-per-tile
+form for small launches (phz_control.h, tanh_layer_split and policy_team).
+
+- The split layers' error against the MLP in 64 bits is no larger than the f32
+  MFMA's on the same weights and inputs. Weights with one value that a bf16
+  piece cannot hold (1e-40) take the f32 kernel and change nothing else by more
+  than 1e-40; infinite weights take it too.
+- The two forms give the same bits, at ragged widths, two output blocks, wide
+  inputs, partial tiles and a single world.
+"""
+import dataclasses
+
+import numpy as np
+import pytest
+
+from phyz_amd import workloads as W
+from phyz_amd.policy import QMinus
+from phyz_amd.sim import from_control_loop
+
+pytestmark = pytest.mark.gpu
+
+
+def _sim(hidden, n, extra=0, noise=0.0):
+    cl = W.control_loop(hidden)
+    obs = list(cl.spec.obs) + [QMinus(6 + k % 8, 0.1 * k) for k in range(extra)]
+    spec = dataclasses.replace(cl.spec, obs=obs, input_noise=[noise] * len(obs), history_steps=3)
+    cl = dataclasses.replace(cl, spec=spec, weights=np.zeros(spec.n_weights()))
+    sim = from_control_loop(cl, "f32", nworld=n)
+    q, v, _, _ = cl.base.initial_state(n)
+    sim.load_states(q, v)
+    return cl, sim
+
+
+def _weights(spec, seed, scale):
+    i, h, o = spec.n_in(), spec.hidden, spec.n_out()
+    rng = np.random.default_rng(seed)
+    parts = [rng.normal(size=(h, i)) / np.sqrt(i), 0.1 * rng.normal(size=h), rng.normal(size=(h, h)) / np.sqrt(h),
+             0.1 * rng.normal(size=h), rng.normal(size=(o, h)) / np.sqrt(h), 0.1 * rng.normal(size=o)]
+    return [(scale * p).astype(np.float32).astype(np.float64) for p in parts]
+
+
+def _flat(parts):
+    return np.concatenate([p.ravel() for p in parts])
+
+
+@pytest.mark.parametrize("hidden,scale", [(32, 1.0), (48, 0.2), (100, 3.0), (256, 1.0), (256, 0.05)])
+def test_split_error_is_not_larger(hidden, scale):
+    err = {}
+    for form in ("f32", "split"):
+        cl, sim = _sim(hidden, 4000)
+        w = _weights(cl.spec, 5, scale)
+        if form == "f32":
+            w[2][0, 0] = 1e-40
+        sim.set_policy_weights(_flat(w))
+        sim.set_policy_std(np.full(8, 1e-30))  # the action is the mean
+        sim.run_policy(0)
+        obs, out = sim.readback_policy_history(0, 1)
+        h = np.tanh(np.tanh(obs[0] @ w[0].T + w[1]) @ w[2].T + w[3])
+        want = h @ w[4].T + w[5]
+        err[form] = np.linalg.norm(out[0][:, :8] - want) / np.linalg.norm(want)
+    print(f"hidden {hidden} scale {scale}: {err}", flush=True)
+    assert err["split"] <= err["f32"]
+
+
+@pytest.mark.parametrize("hidden,n,extra", [(32, 1, 0), (40, 50, 3), (64, 4000, 40), (256, 33, 0), (256, 4097, 4)])
+def test_team_same_bits(hidden, n, extra, monkeypatch):
+    outs = []
+    for team in ("0", "1"):
+        monkeypatch.setenv("PHZ_POLICY_TEAM", team)
+        cl, sim = _sim(hidden, n, extra, 0.02)
+        sim.set_policy_weights(_flat(_weights(cl.spec, 6, 1.0)))
+        sim.seed_policy(9)
+        assert sim.control_kernel_info("policy")["block"] == (256 if team == "1" else 64)
+        sim.rollout(0, 3, 2, False)
+        outs.append(sim.readback_policy_history(0, 3) + (sim.readback_targets(),) + sim.readback_states())
+    for x, y in zip(*outs):
+        assert np.isfinite(x).all() and np.array_equal(x, y)
+
+
+def test_weights_out_of_range_take_f32_and_back():
+    cl, sim = _sim(64, 100)
+    w = _weights(cl.spec, 7, 1.0)
+    sim.set_policy_std(np.full(8, 1e-30))
+    got = []
+    for k, first in enumerate((w[2][0, 0], np.inf, w[2][0, 0])):
+        w[2][0, 0] = first
+        sim.set_policy_weights(_flat(w))
+        sim.run_policy(k)
+        obs, out = sim.readback_policy_history(k, k + 1)
+        h = np.tanh(np.tanh(obs[0] @ w[0].T + w[1]) @ w[2].T + w[3])
+        got.append(out[0][:, :8])
+        assert np.abs(got[-1] - (h @ w[4].T + w[5])).max() < 1e-5
+    assert np.array_equal(got[0], got[2])
