@@ -20,8 +20,8 @@
 //               (tanh_layer_split). Only the per-world prologue (input noise)
 //               and epilogue (Gaussian sample, log-prob, PD targets) go
 //               through LDS, because each world's random stream is sequential
-//               and lives in one lane. Small launches give a tile of 16
-//               worlds to a workgroup of four waves instead (policy_team).
+//               and lives in one lane. Small launches give a tile of 16 or 32
+//               worlds to a workgroup of 4 or 8 waves instead (policy_team).
 #pragma once
 
 namespace phz {
@@ -637,16 +637,20 @@ template <class P, class T> __device__ __forceinline__ void policy_wave(const Po
 // ── small launches: a tile of 16 CB worlds to a workgroup of TW waves ──
 // One wave per tile leaves most SIMDs idle when a launch has few tiles, and
 // the launch then lasts as long as one wave's stream (29-256-256-8: 40 us at
-// 64 worlds, 44 at 16384; here 16 and 39). Here wave k computes the hidden neurons of blocks
+// 64 worlds, 44 at 16384; here 16 and 29). Here wave k computes the hidden neurons of blocks
 // k * BPW .. of both hidden layers for the whole tile, and passes them to the
 // others through LDS, already split into bf16 pieces and laid out as B
 // fragments. The streams' raw draws are one lane's work per world, the
 // Box-Muller transforms are spread over every lane. Every sum runs in
 // policy_wave's order: the two give the same bits.
 //
-// LDS: the draws (8 bytes each, later the hidden pieces: KB2 x 3 x CB x 1 KB),
+// LDS: the draws (8 bytes each, kTeamDraws normals at a time, later the hidden pieces: KB2 x 3 x CB x 1 KB),
 // the input tile [world][XS], the means [world][MS] and the actions' normals.
-template <class P> constexpr int team_draws() { return 2 * (noised_inputs<P>() + P::NO) * 16 * P::CB * 8; }
+constexpr int kTeamDraws = 40;  // normals drawn at a time
+template <class P> constexpr int team_draws() {
+  const int n = noised_inputs<P>() + P::NO;
+  return 2 * (n < kTeamDraws ? n : kTeamDraws) * 16 * P::CB * 8;
+}
 template <class P> constexpr int team_pieces() { return ((P::NHB + 1) / 2) * 3 * P::CB * 1024; }
 template <class P> constexpr int team_front() {
   return team_draws<P>() > team_pieces<P>() ? team_draws<P>() : team_pieces<P>();
@@ -713,33 +717,37 @@ template <class P, class T> __device__ __forceinline__ void policy_team(const Po
   float z[NO];
   if (sampler) sample_state<P, T>(a, w0 + tid, base, z);
 
-  // Raw draws in stream order (inputs, then actions) by one lane per world of
-  // the first wave; the other waves stage the observation rows.
-  if (tid < W) {
-    const int my = w0 + tid;
-    u64 rs = my < a.nworld ? a.rng[my] : 1;
-#pragma unroll 4
-    for (int d = 0; d < 2 * ND; d++) draws[d * W + tid] = xorshift64(rs);
-    if (my < a.nworld) a.rng[my] = rs;
-  }
   for (int e = tid; e < 16 * KU * W; e += 64 * TW) {
     const int i = e / W, w = e % W;
     x[w * XS + i] = i < NI && w0 + w < a.nworld ? a.obs[(size_t)i * S + w0 + w] : 0.0f;
   }
-  __syncthreads();
-  for (int e = tid; e < ND * W; e += 64 * TW) {
-    const int d = e / W, w = e % W;
-    const u64 x1 = draws[(2 * d) * W + w], x2 = draws[(2 * d + 1) * W + w];
-    const float n = (float)policy_transform(uniform_of(x1), turns_of(x2));
-    if (d < NN) {
-      const int i = P::noised[d];
-      const float xi = fmaf(P::scale[d], n, x[w * XS + i]);
-      x[w * XS + i] = xi;
-      if (w0 + w < a.nworld) a.obs[(size_t)i * S + w0 + w] = xi;
-    } else {
-      nact[(d - NN) * W + w] = n;
+  // Raw draws in stream order (inputs, then actions) by one lane per world of
+  // the first wave, then their transforms on every lane.
+  u64 rs = 1;
+  if (sampler) rs = a.rng[w0 + tid];
+  for (int d0 = 0; d0 < ND; d0 += kTeamDraws) {
+    const int nd = ND - d0 < kTeamDraws ? ND - d0 : kTeamDraws;
+    if (d0 > 0) __syncthreads();  // the transforms of the draws before are done
+    if (tid < W) {
+#pragma unroll 4
+      for (int d = 0; d < 2 * nd; d++) draws[d * W + tid] = xorshift64(rs);
+    }
+    __syncthreads();
+    for (int e = tid; e < nd * W; e += 64 * TW) {
+      const int d = e / W, w = e % W, k = d0 + d;
+      const u64 x1 = draws[(2 * d) * W + w], x2 = draws[(2 * d + 1) * W + w];
+      const float n = (float)policy_transform(uniform_of(x1), turns_of(x2));
+      if (k < NN) {
+        const int i = P::noised[k];
+        const float xi = fmaf(P::scale[k], n, x[w * XS + i]);
+        x[w * XS + i] = xi;
+        if (w0 + w < a.nworld) a.obs[(size_t)i * S + w0 + w] = xi;
+      } else {
+        nact[(k - NN) * W + w] = n;
+      }
     }
   }
+  if (sampler) a.rng[w0 + tid] = rs;
   __syncthreads();
 
   const int r = lane & 15, g = lane >> 4;

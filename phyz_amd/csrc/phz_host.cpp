@@ -1296,15 +1296,14 @@ std::string gen_obs_source(const ModelD& m, const PolicyD* p, bool f64) {
 }
 
 // Policy kernel: widths, action wiring and noise scales compiled in.
-// two_waves: as gen_source's, two resident waves per SIMD. team: a workgroup
-// of kTeamWaves waves per 16 worlds (policy_team).
-constexpr int kTeamWaves = 4;
-std::string gen_policy_source(const PolicyD& p, int npd, bool f64, bool two_waves = false, bool team = false) {
+// two_waves: as gen_source's, two resident waves per SIMD. team > 0: a
+// workgroup of 4 team waves per 16 team worlds (policy_team).
+std::string gen_policy_source(const PolicyD& p, int npd, bool f64, bool two_waves = false, int team = 0) {
   const std::string T = f64 ? "double" : "float";
   std::string s = kDeviceSrc;
   s += "\n";
   s += kControlSrc;
-  const int cb = team ? 1 : p.cb();
+  const int cb = team ? team : p.cb();
   // Two-wave builds park tiles of layer 1 in LDS, up to 16 KB per wave (8
   // waves of 18 KB a CU) instead of spilling them: at hidden 256, 284 -> 52 B
   // of scratch per lane, 155 -> 149 us.
@@ -1314,7 +1313,7 @@ std::string gen_policy_source(const PolicyD& p, int npd, bool f64, bool two_wave
   o << "\n// ---- policy shape ----\nstruct Pol {\n";
   o << "  static constexpr int NI = " << p.n_in << ", NH = " << p.hidden << ", NO = " << p.n_out << ", NHB = " << p.nhb()
     << ", NOB = " << p.nob() << ", KU = " << p.ku() << ", CB = " << cb << ", NPD = " << npd << ", LDS = " << lds
-    << ", TW = " << kTeamWaves << ", PARK = " << park << ";\n";
+    << ", TW = " << 4 * std::max(team, 1) << ", PARK = " << park << ";\n";
   o << "  static constexpr bool SPLIT = " << (p.split ? "true" : "false") << ";\n";
   std::vector<int> noised;  // the inputs with noise, in order
   for (int k = 0; k < p.n_in; k++) if (p.noise[k] != 0.0) noised.push_back(k);
@@ -1330,7 +1329,7 @@ std::string gen_policy_source(const PolicyD& p, int npd, bool f64, bool two_wave
     << ";\n};\n";
   s += o.str();
   if (team) {
-    s += "extern \"C\" __global__ void __launch_bounds__(" + std::to_string(64 * kTeamWaves) + ") phz_policy(phz::PolicyArgs a) {\n";
+    s += "extern \"C\" __global__ void __launch_bounds__(" + std::to_string(256 * team) + ") phz_policy(phz::PolicyArgs a) {\n";
     s += "  __shared__ __align__(16) char lds[phz::team_lds_bytes<Pol>()];\n";
     s += "  if (threadIdx.x < 64) phz::fill_tables(threadIdx.x);\n  __syncthreads();\n";
     s += "  phz::policy_team<Pol, " + T + ">(a, lds);\n}\n";
@@ -1430,7 +1429,7 @@ struct phz_sim {
   uint64_t ctl_epoch = 1;       // bumped when the model, PD table or policy spec changes
   bool policy_on = false;
   PolicyD pol;
-  bool pol_team = false;        // pol_k is the workgroup-per-tile form
+  int pol_team = 0;             // > 0: pol_k is the workgroup-per-tile form, 16 pol_team worlds a tile
   float* pw = nullptr;          // weight fragments and biases
   float* pstd = nullptr;        // [n_out]
   float* obs_hist = nullptr;    // [history][n_in][stride]
@@ -1669,16 +1668,24 @@ struct phz_sim {
   float* obs_row(uint32_t step) const { return obs_hist + (size_t)step * pol.n_in * stride; }
   float* out_row(uint32_t step) const { return out_hist + (size_t)step * (pol.n_out + 1) * stride; }
 
-  // Whether a policy launch of this size runs the workgroup-per-tile kernel:
-  // up to four 16-world tiles per CU. us per launch, one wave per tile against
-  // it (29 inputs, 8 actions): hidden 256, 64 worlds 40 / 16, 4096 41 / 18,
-  // 8192 42 / 23, 16384 44 / 39, 24576 46 / 51; hidden 64, 4096 26 / 13, 16384
-  // 27 / 18, 24576 28 / 25, 65536 31 / 49. PHZ_POLICY_TEAM=0|1 forces it off or
-  // on (tests, tuning).
-  bool team_pays() const {
-    if (!pol.split) return false;
-    if (const char* e = std::getenv("PHZ_POLICY_TEAM")) return e[0] == '1';
-    return ((long)nworld + 15) / 16 <= 4L * std::max(feat.cus, 1);
+  // The workgroup-per-tile policy kernel's tile for a launch of this size, in
+  // 16-world columns; 0: one wave per tile. It runs up to four columns per CU,
+  // as 16-world tiles (4 waves) up to one per CU, beyond that and for wide
+  // nets as 32-world tiles (8 waves), which read the weights half as often.
+  // us per launch, one wave per tile / 16-world / 32-world tiles:
+  //   29 inputs, hidden 256, 8 actions: 64 worlds 40 / 15.8 / 18.0, 4096 41 /
+  //   17.9 / 19.1, 8192 42 / 23.0 / 20.6, 16384 44 / 38.4 / 29.2, 32768 49 /
+  //   67 / 51.5; hidden 64: 4096 26 / 12.2 / 13.8, 16384 27 / 17.6 / 18.0,
+  //   24576 28 / 24.6 / 28.8;
+  //   128, 256, 32: 4096 79 / 36.4 / 38.0, 8192 81 / 46.2 / 40.0, 16384 86 /
+  //   85.7 / 70.2.
+  // PHZ_POLICY_TEAM=0|1|2 forces the form (tests, tuning).
+  int team_columns() const {
+    if (!pol.split) return 0;
+    if (const char* e = std::getenv("PHZ_POLICY_TEAM")) return std::max(0, std::min(2, std::atoi(e)));
+    const long columns = ((long)nworld + 15) / 16, cus = std::max(feat.cus, 1);
+    if (columns > 4 * cus) return 0;
+    return columns > cus || pol.n_in + pol.n_out > 64 ? 2 : 1;
   }
   // Compile (and with `load`, load) the FK/observation or the policy kernel
   // for the current configuration epoch.
@@ -1690,7 +1697,7 @@ struct phz_sim {
       k.reset();
     }
     if (!k.code) {
-      if (policy_kernel) pol_team = team_pays();
+      if (policy_kernel) pol_team = team_columns();
       const std::string src = policy_kernel ? gen_policy_source(pol, feat.npd, f64, false, pol_team)
                                             : gen_obs_source(model, policy_on ? &pol : nullptr, f64);
       std::string e;
@@ -1735,12 +1742,13 @@ struct phz_sim {
     return hip_ok(hipModuleLaunchKernel(obs_k.fn, grid, 1, 1, 64, 1, 1, 0, stream, params, nullptr), "obs kernel launch");
   }
   bool launch_policy(uint32_t step) {
-    const int wpw = pol_team ? 16 : 16 * pol.cb();
+    const int wpw = 16 * (pol_team ? pol_team : pol.cb());
     PolicyArgs a{pw, pw + pol.off_w2(), pw + pol.off_w3(), pw + pol.off_bias(), pstd, obs_row(step), out_row(step),
                  prng, pz, pbase, targets, nworld, stride};
     void* params[] = {&a};
     const unsigned grid = (unsigned)((nworld + wpw - 1) / wpw);
-    return hip_ok(hipModuleLaunchKernel(pol_k.fn, grid, 1, 1, pol_team ? 64 * kTeamWaves : 64, 1, 1, 0, stream, params, nullptr),
+    return hip_ok(hipModuleLaunchKernel(pol_k.fn, grid, 1, 1, pol_team ? 256 * (unsigned)pol_team : 64, 1, 1, 0, stream,
+                                        params, nullptr),
                   "policy kernel launch");
   }
   // Everything run_policy needs, checked on the host (mod.rs:1209-1231).
@@ -2782,9 +2790,9 @@ int phz_control_kernel_info(phz_sim* s, int which, int64_t* info) {
   info[1] = remark_value(log, "AGPRs:");
   info[2] = remark_value(log, "SGPRs:");
   info[3] = remark_value(log, "ScratchSize [bytes/lane]:");
-  const bool team = which == 1 && s->pol_team;
-  info[4] = team ? 64 * kTeamWaves : 64;
-  info[5] = team ? 16 : which == 1 ? 16 * s->pol.cb() : 64;
+  const int team = which == 1 ? s->pol_team : 0;
+  info[4] = team ? 256 * team : 64;
+  info[5] = which == 1 ? 16 * (team ? team : s->pol.cb()) : 64;
   return 0;
 }
 

@@ -5,7 +5,7 @@ form for small launches (phz_control.h, tanh_layer_split and policy_team).
   MFMA's on the same weights and inputs. Weights with one value that a bf16
   piece cannot hold (1e-40) take the f32 kernel and change nothing else by more
   than 1e-40; infinite weights take it too.
-- The two forms give the same bits, at ragged widths, two output blocks, wide
+- The three forms give the same bits, at ragged widths, two output blocks, wide
   inputs, partial tiles and a single world.
 """
 import dataclasses
@@ -62,19 +62,20 @@ def test_split_error_is_not_larger(hidden, scale):
     assert err["split"] <= err["f32"]
 
 
-@pytest.mark.parametrize("hidden,n,extra", [(32, 1, 0), (40, 50, 3), (64, 4000, 40), (256, 33, 0), (256, 4097, 4)])
+@pytest.mark.parametrize("hidden,n,extra", [(32, 1, 0), (40, 50, 3), (64, 4000, 40), (256, 33, 0), (256, 4097, 4),
+                                             (256, 70, 99)])
 def test_team_same_bits(hidden, n, extra, monkeypatch):
     outs = []
-    for team in ("0", "1"):
+    for team in ("0", "1", "2"):
         monkeypatch.setenv("PHZ_POLICY_TEAM", team)
         cl, sim = _sim(hidden, n, extra, 0.02)
         sim.set_policy_weights(_flat(_weights(cl.spec, 6, 1.0)))
         sim.seed_policy(9)
-        assert sim.control_kernel_info("policy")["block"] == (256 if team == "1" else 64)
+        assert sim.control_kernel_info("policy")["block"] == {"0": 64, "1": 256, "2": 512}[team]
         sim.rollout(0, 3, 2, False)
         outs.append(sim.readback_policy_history(0, 3) + (sim.readback_targets(),) + sim.readback_states())
-    for x, y in zip(*outs):
-        assert np.isfinite(x).all() and np.array_equal(x, y)
+    for x, y, z in zip(*outs):
+        assert np.isfinite(x).all() and np.array_equal(x, y) and np.array_equal(x, z)
 
 
 def test_weights_out_of_range_take_f32_and_back():
