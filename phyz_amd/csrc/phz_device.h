@@ -2521,7 +2521,12 @@ template <class M, class T, int G> __device__ __forceinline__ void run_group(con
       __syncthreads();
     }
     for (int s = 0; s < n; s++) {
-      const bool last = (s == n - 1) && a.write_contacts && live;
+      int left = n - 1 - s;
+      // The partitioned small trees: without this the compiler peels the last
+      // step, whose copy it contracts differently from the loop's, and a
+      // span's bits would depend on how it is cut into launches (the f32 ant).
+      if constexpr (M::PMODE == 2 && M::NB < 14) asm volatile("" : "+s"(left));
+      const bool last = left == 0 && a.write_contacts && live;
       step_group<M, T, G>(q, v, ctrl, qdd, tgt, rng, rows, S, last, lds, lane, tr, s + 1 < n);
     }
   }

@@ -174,6 +174,7 @@ struct Features {
   // for the partition plan.
   int wgs = 0, cus = 256;
   bool f64 = false;  // the sim's precision (the planner keeps f64 subtrees one per wave)
+  bool lane_small_tree = false;  // no partition of a tree of fewer than 14 bodies (phz_sim::compile)
   bool host_only = false;  // a sim without a device (device ordinal -1): code generation only
   // Terms of the CPU model that the device body table has no slots for
   // (joint.rs:27-104, model.rs:18-82): the soft position limit and dry friction
@@ -300,7 +301,18 @@ Plan plan_partition(const ModelD& m, const Features& f) {
   }
   const bool forced = want == "1" || want == "2";
   if (parts.size() < 2) return lane_per_world();
-  if (mode == 2 && !forced && nb < 14) return lane_per_world();
+  // Trees of fewer than 14 bodies (the ants) are partitioned in f32 launches of
+  // up to three workgroups per CU, where the waves per world group fill SIMDs
+  // that a lane per world leaves idle or lightly loaded; their kernels hold at
+  // most 256 registers, so workgroups share SIMDs and none waits for a further
+  // round (phz_sim::compile takes the lane plan back where one does not).
+  // Measured, us per 100-step launch, lane per world / 4 waves: ant 64 worlds
+  // 447 / 259, 16384 465 / 278, 32768 472 / 362, 49152 485 / 446, 65536 502 /
+  // 637; with PD servos 427 / 230 to 464 / 423 at 49152; MJCF ant 807 / 325,
+  // 826 / 357, 836 / 493, 865 / 779, 882 / 930. f64 keeps one lane per world.
+  const bool small_tree = mode == 2 && nb < 14 && !f.f64;
+  if (mode == 2 && !forced && nb < 14 && (f.f64 || f.lane_small_tree || f.wgs > 3 * std::max(f.cus, 1)))
+    return lane_per_world();
   // Waves per world group, from a model of a step's length in body weights
   // (a hinge, slide or ball body 4, a free body 8, a body without DOFs 2):
   //  - A wave's own bodies run passes 1-3 in its own instruction stream; wave 0
@@ -344,7 +356,7 @@ Plan plan_partition(const ModelD& m, const Features& f) {
   auto cost = [&](const std::vector<double>& load) {
     const int ng = (int)load.size(), cus = std::max(f.cus, 1);
     const long per_cu = std::max(1, (f.wgs + cus - 1) / cus);
-    const long conc = ng <= 4 ? 4 / ng : 1;
+    const long conc = (ng <= 4 ? 4 / ng : 1) * (small_tree ? 4 : 1);
     const long rounds = (per_cu + conc - 1) / conc;
     double simd[4] = {0, 0, 0, 0};
     for (int k = 0; k < ng; k++) simd[k % 4] += load[k] + pass1 + (k == 0 ? tcontact : 0.0);
@@ -354,6 +366,7 @@ Plan plan_partition(const ModelD& m, const Features& f) {
   // dropped, no plan of exactly three groups), as group -> part indices.
   auto pack = [&](int cap) {
     const int n = (int)parts.size();
+    cap = std::min(cap, n);  // more groups than parts are empty ones: the same plans
     std::vector<std::vector<int>> best;
     double best_cost = -1;
     auto consider = [&](const std::vector<int>& owner) {
@@ -1505,7 +1518,17 @@ struct phz_sim {
     if (code) return true;
     std::string e;
     int ng = 1;
-    const std::string src = gen_source(model, feat, f64, &ng, &lanes);
+    feat.lane_small_tree = false;
+    std::string src = gen_source(model, feat, f64, &ng, &lanes);
+    if (ng > 1 && model.nb < 14 && !f64 && feat.wgs > feat.cus) {
+      // The plan of a small tree counts on two waves per SIMD (plan_partition).
+      std::string e2;
+      const auto co = compile_source(src, Build::Reassoc, e2);
+      if (co && remark_value(co->log, "VGPRs:") + std::max<int64_t>(remark_value(co->log, "AGPRs:"), 0) > 256) {
+        feat.lane_small_tree = true;
+        src = gen_source(model, feat, f64, &ng, &lanes);
+      }
+    }
     block = 64 * ng;
     if (const char* dump = std::getenv("PHZ_DUMP_SOURCE")) {
       std::ofstream out(dump);
