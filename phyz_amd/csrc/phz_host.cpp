@@ -14,6 +14,7 @@
 #include <hip/hiprtc.h>
 #include <sys/stat.h>
 #include <unistd.h>
+#include <xmmintrin.h>
 
 #include <algorithm>
 #include <chrono>
@@ -41,9 +42,16 @@ static const char* const kControlSrc =
 #include "phz_control_src.inc"
     ;
 
+constexpr int kPhzRowParts = 3;
+struct PhzRowParts {  // must match phz_io.hip
+  void* soa[kPhzRowParts];
+  void* rows[kPhzRowParts];
+  int width[kPhzRowParts];
+  int parts, first, count, stride;
+};
 extern "C" {
-hipError_t phz_io_pack(const double* src, void* dst, int nworld, int width, int stride, int f64, hipStream_t s);
-hipError_t phz_io_unpack(const void* src, double* dst, int nworld, int width, int stride, int f64, hipStream_t s);
+hipError_t phz_io_rows_out(const PhzRowParts* p, int soa_f64, int rows_f64, hipStream_t s);
+hipError_t phz_io_rows_in(const PhzRowParts* p, int f64, hipStream_t s);
 hipError_t phz_io_zero(void* dst, size_t bytes, hipStream_t s);
 hipError_t phz_io_seed(uint64_t* rng, uint64_t seed, int nworld, hipStream_t s);
 hipError_t phz_io_copy(void* dst, const void* src, size_t bytes, hipStream_t s);
@@ -1117,6 +1125,28 @@ struct PolicyD {
   }
 };
 
+// Rows between a caller's f64 array and a staging slot in the array's
+// precision, rounded to nearest with subnormals kept whatever the calling
+// thread's floating-point mode (MXCSR) is, as the device's conversions are.
+__attribute__((noinline)) void convert_loop(bool up, double* host, void* slot, size_t n) {
+  float* f = (float*)slot;
+  if (up)
+    for (size_t k = 0; k < n; k++) f[k] = (float)host[k];
+  else
+    for (size_t k = 0; k < n; k++) host[k] = (double)f[k];
+}
+void convert_rows(bool up, double* host, void* slot, size_t n, bool f64) {
+  if (f64) {
+    if (up) std::memcpy(slot, host, n * 8);
+    else std::memcpy(host, slot, n * 8);
+    return;
+  }
+  const unsigned mode = _mm_getcsr();
+  _mm_setcsr(0x1f80);
+  convert_loop(up, host, slot, n);
+  _mm_setcsr(mode);
+}
+
 // The bf16 nearest x (ties to even), as its 16 bits; x finite.
 uint16_t bf16_bits(float x) {
   uint32_t u;
@@ -1418,8 +1448,14 @@ struct phz_sim {
   void *ext_buf = nullptr, *imp_buf = nullptr, *hf_buf = nullptr;  // impulse solver state; heightfield nodes (f64)
   size_t hf_cap = 0;                                                // node capacity of hf_buf
   uint64_t* rng = nullptr;
-  double* staging = nullptr;
-  size_t staging_bytes = 0;
+  // Pinned host memory that state rows pass through, kSlots slots used in turn
+  // (move_rows): at most 4 x 512 KB, or 4 x 64 worlds' rows where those are more.
+  static constexpr int kSlots = 4;
+  static constexpr size_t kSlotBytes = size_t(512) << 10;
+  char* pin = nullptr;
+  size_t pin_slot = 0;
+  hipEvent_t pin_ev[kSlots] = {};
+  bool pin_busy[kSlots] = {};  // a kernel may still use the slot: wait for its event first
   std::shared_ptr<CodeObject> code;
   hipModule_t module = nullptr;
   hipFunction_t fn = nullptr;
@@ -1484,34 +1520,122 @@ struct phz_sim {
     if (!hip_ok(hipMalloc(p, std::max<size_t>(bytes, 256)), what)) return false;
     return hip_ok(phz_io_zero(*p, std::max<size_t>(bytes, 256), stream), what);
   }
-  bool ensure_staging(size_t bytes) {
-    if (bytes <= staging_bytes) return true;
-    // A pack or unpack kernel queued on the stream may still read the old buffer.
-    if (staging && !hip_ok(hipStreamSynchronize(stream), "staging sync")) return false;
-    if (staging) hipFree(staging);
-    staging = nullptr;
-    staging_bytes = 0;
-    if (!hip_ok(hipMalloc((void**)&staging, bytes), "staging alloc")) return false;
-    staging_bytes = bytes;
+  bool ensure_pin(size_t slot) {
+    for (auto& e : pin_ev)
+      if (!e && !hip_ok(hipEventCreateWithFlags(&e, hipEventDisableTiming), "staging event")) return false;
+    if (slot <= pin_slot) return true;
+    // A kernel queued on the stream may still use the old memory.
+    if (pin && !hip_ok(hipStreamSynchronize(stream), "staging sync")) return false;
+    if (pin) (void)hipHostFree(pin);
+    pin = nullptr;
+    pin_slot = 0;
+    for (bool& b : pin_busy) b = false;
+    if (!hip_ok(hipHostMalloc((void**)&pin, slot * kSlots, hipHostMallocDefault), "staging alloc")) return false;
+    pin_slot = slot;
     return true;
   }
-  // host [nworld][width] f64 -> device SoA
+  // Poll for up to 200 us before blocking: a blocking wait wakes the host
+  // about 10 us after the work ends.
+  template <class Query, class Block> bool wait(Query query, Block block, const char* what) {
+    const auto t0 = std::chrono::steady_clock::now();
+    for (;;) {
+      const hipError_t e = query();
+      if (e == hipSuccess) return true;
+      if (e != hipErrorNotReady) return hip_ok(e, what);
+      if (std::chrono::steady_clock::now() - t0 > std::chrono::microseconds(200)) break;
+    }
+    return hip_ok(block(), what);
+  }
+  bool wait_event(hipEvent_t ev, const char* what) {
+    return wait([&] { return hipEventQuery(ev); }, [&] { return hipEventSynchronize(ev); }, what);
+  }
+  bool wait_stream(const char* what) {
+    return wait([&] { return hipStreamQuery(stream); }, [&] { return hipStreamSynchronize(stream); }, what);
+  }
+  struct Rows {
+    void* soa;         // device SoA [width][stride]
+    double* host;      // [groups][nworld][width]
+    int width;
+    size_t step = 0;   // bytes from one group's SoA to the next's
+  };
+  // Rows between host arrays and device SoAs through the pinned slots: the
+  // host converts a slot's worlds (f64 <-> the array's precision, as the
+  // device's conversion rounds) while kernels move the other slots' over PCIe.
+  // Pageable hipMemcpys of f64 rows did 8-17 GB/s on readback (less into
+  // memory not yet touched) and 30 GB/s on upload; this host core converts at
+  // about 80 GB/s from and to cache. us per call, copies / slots: readback of
+  // 65536 x 14 f32 values 1767 / 168 (into touched memory 451 / 165), of
+  // 131072 x 28 3355 / 1644 (1653 / 690), of 8192 x 28 144 / 59, of 96 x 4 f64
+  // 52 / 16; load of 65536 x 21 371 / 231, of 96 x 6 29 / 20. Small rows gain
+  // from one launch and one wait for q and v together, large ones from the
+  // bytes; where the caller's memory is untouched its page faults remain.
+  bool move_rows(bool up, const Rows* rows, int nrows, int groups, bool is_f64, const char* what) {
+    Rows part[kPhzRowParts];
+    size_t off[kPhzRowParts] = {};
+    int np = 0;
+    size_t per_world = 0;
+    const size_t E = is_f64 ? 8 : 4, W = (size_t)nworld;
+    for (int k = 0; k < nrows; k++)
+      if (rows[k].host && rows[k].width > 0) {
+        part[np++] = rows[k];
+        per_world += rows[k].width * E;
+      }
+    if (np == 0 || W == 0 || groups <= 0) return true;
+    // A slot holds whole tiles of 64 worlds, each part from a 256-byte boundary.
+    const size_t pad = 256 * kPhzRowParts, tiles = (W + 63) / 64, tile_bytes = 64 * per_world;
+    const size_t fit = std::max<size_t>(1, kSlotBytes > pad ? (kSlotBytes - pad) / tile_bytes : 1);
+    const size_t cw = 64 * std::min(tiles, fit), per_group = (W + cw - 1) / cw, chunks = per_group * groups;
+    if (!ensure_pin((cw * per_world + pad + 4095) & ~size_t(4095))) return false;
+    for (int k = 1; k < np; k++) off[k] = (off[k - 1] + cw * part[k - 1].width * E + 255) & ~size_t(255);
+    auto launch = [&](size_t i) {
+      const size_t g = i / per_group, first = i % per_group * cw, slot = i % kSlots;
+      PhzRowParts p{};
+      for (int k = 0; k < np; k++) {
+        p.soa[k] = (char*)part[k].soa + g * part[k].step;
+        p.rows[k] = pin + slot * pin_slot + off[k];
+        p.width[k] = part[k].width;
+      }
+      p.parts = np;
+      p.first = (int)first;
+      p.count = (int)std::min(cw, W - first);
+      p.stride = stride;
+      pin_busy[slot] = true;
+      return hip_ok(up ? phz_io_rows_in(&p, is_f64, stream) : phz_io_rows_out(&p, is_f64, is_f64, stream), what) &&
+             hip_ok(hipEventRecord(pin_ev[slot], stream), what);
+    };
+    auto convert = [&](size_t i) {
+      const size_t g = i / per_group, first = i % per_group * cw, n = std::min(cw, W - first), slot = i % kSlots;
+      for (int k = 0; k < np; k++)
+        convert_rows(up, part[k].host + (g * W + first) * part[k].width, pin + slot * pin_slot + off[k],
+                     n * part[k].width, is_f64);
+    };
+    if (up) {
+      for (size_t i = 0; i < chunks; i++) {
+        const size_t slot = i % kSlots;
+        if (pin_busy[slot] && !wait_event(pin_ev[slot], what)) return false;
+        convert(i);
+        if (!launch(i)) return false;
+      }
+      return true;
+    }
+    for (size_t issued = 0, done = 0; done < chunks; done++) {
+      for (; issued < chunks && issued < done + kSlots; issued++)
+        if (!launch(issued)) return false;
+      if (!wait_event(pin_ev[done % kSlots], what)) return false;
+      pin_busy[done % kSlots] = false;
+      convert(done);
+    }
+    return true;
+  }
+  // host [nworld][width] f64 -> device SoA; the host array is free on return.
   bool upload_rows(const double* host, void* dst, int width, const char* what) {
-    if (width <= 0) return true;
-    const size_t bytes = (size_t)nworld * width * sizeof(double);
-    if (!ensure_staging(bytes)) return false;
-    if (!hip_ok(hipMemcpyAsync(staging, host, bytes, hipMemcpyHostToDevice, stream), what)) return false;
-    return hip_ok(phz_io_pack(staging, dst, nworld, width, stride, f64 ? 1 : 0, stream), what);
+    const Rows r{dst, const_cast<double*>(host), width};
+    return move_rows(true, &r, 1, 1, f64, what);
   }
   // elem: 1 = f64, 0 = f32 source; -1 = the sim's precision.
   bool download_rows(const void* src, double* host, int width, const char* what, int elem = -1) {
-    if (width <= 0) return true;
-    const size_t bytes = (size_t)nworld * width * sizeof(double);
-    if (!ensure_staging(bytes)) return false;
-    const int src_f64 = elem < 0 ? (f64 ? 1 : 0) : elem;
-    if (!hip_ok(phz_io_unpack(src, staging, nworld, width, stride, src_f64, stream), what)) return false;
-    if (!hip_ok(hipMemcpyAsync(host, staging, bytes, hipMemcpyDeviceToHost, stream), what)) return false;
-    return hip_ok(hipStreamSynchronize(stream), what);
+    const Rows r{const_cast<void*>(src), host, width};
+    return move_rows(false, &r, 1, 1, elem < 0 ? f64 : elem != 0, what);
   }
 
   bool compile() {
@@ -1864,8 +1988,11 @@ struct phz_sim {
       obs_k.reset();
       pol_k.reset();
       free_policy_buffers();
-      for (void* p : {q, v, ctrl, qdd, targets, rows, (void*)rng, (void*)staging, kin, hq, hv, ext_buf, imp_buf, hf_buf})
+      for (void* p : {q, v, ctrl, qdd, targets, rows, (void*)rng, kin, hq, hv, ext_buf, imp_buf, hf_buf})
         if (p) hipFree(p);
+      if (pin) (void)hipHostFree(pin);
+      for (hipEvent_t e : pin_ev)
+        if (e) (void)hipEventDestroy(e);
       if (stream) hipStreamDestroy(stream);
     }
   }
@@ -2358,14 +2485,14 @@ int phz_load_states(phz_sim* s, const double* q, const double* v, const double* 
   if (!q || !v) return s->fail("null q or v");
   if (!s->has_device()) return s->fail("host-only sim has no device buffers");
   if (!set_device(s)) return 1;
-  if (!s->upload_rows(q, s->q, s->model.nq, "upload q") || !s->upload_rows(v, s->v, s->model.nv, "upload v")) return 1;
-  if (ctrl) {
-    if (!s->upload_rows(ctrl, s->ctrl, s->nctrl(), "upload ctrl")) return 1;
-  } else if (!s->hip_ok(phz_io_zero(s->ctrl, (size_t)s->nctrl() * s->stride * s->esize(), s->stream), "zero ctrl")) {
+  const phz_sim::Rows rows[3] = {{s->q, const_cast<double*>(q), s->model.nq},
+                                 {s->v, const_cast<double*>(v), s->model.nv},
+                                 {s->ctrl, const_cast<double*>(ctrl), s->nctrl()}};
+  if (!s->move_rows(true, rows, 3, 1, s->f64, "upload states")) return 1;
+  if (!ctrl && !s->hip_ok(phz_io_zero(s->ctrl, (size_t)s->nctrl() * s->stride * s->esize(), s->stream), "zero ctrl"))
     return 1;
-  }
   if (s->feat.noise && !s->hip_ok(phz_io_seed(s->rng, s->feat.seed, s->nworld, s->stream), "seed rng")) return 1;
-  return s->hip_ok(hipStreamSynchronize(s->stream), "load_states") ? 0 : 1;
+  return s->wait_stream("load_states") ? 0 : 1;
 }
 
 int phz_set_controls(phz_sim* s, const double* ctrl) {
@@ -2374,7 +2501,7 @@ int phz_set_controls(phz_sim* s, const double* ctrl) {
   if (!s->has_device()) return s->fail("host-only sim has no device buffers");
   if (!set_device(s)) return 1;
   if (!s->upload_rows(ctrl, s->ctrl, s->nctrl(), "upload ctrl")) return 1;
-  return s->hip_ok(hipStreamSynchronize(s->stream), "set_controls") ? 0 : 1;
+  return s->wait_stream("set_controls") ? 0 : 1;
 }
 
 int phz_step(phz_sim* s) { return phz_step_many(s, 1); }
@@ -2397,25 +2524,15 @@ int phz_synchronize(phz_sim* s) {
   if (!s) return 1;
   if (!s->has_device()) return 0;
   if (!set_device(s)) return 1;
-  // Poll the stream for up to 200 us before blocking: a blocking wait wakes
-  // the host about 10 us after a short span ends.
-  const auto t0 = std::chrono::steady_clock::now();
-  for (;;) {
-    const hipError_t e = hipStreamQuery(s->stream);
-    if (e == hipSuccess) return 0;
-    if (e != hipErrorNotReady) return s->hip_ok(e, "synchronize") ? 0 : 1;
-    if (std::chrono::steady_clock::now() - t0 > std::chrono::microseconds(200)) break;
-  }
-  return s->hip_ok(hipStreamSynchronize(s->stream), "synchronize") ? 0 : 1;
+  return s->wait_stream("synchronize") ? 0 : 1;
 }
 
 int phz_readback_states(phz_sim* s, double* q, double* v) {
   if (!s) return 1;
   if (!s->has_device()) return s->fail("host-only sim has no device buffers");
   if (!set_device(s)) return 1;
-  if (q && !s->download_rows(s->q, q, s->model.nq, "readback q")) return 1;
-  if (v && !s->download_rows(s->v, v, s->model.nv, "readback v")) return 1;
-  return 0;
+  const phz_sim::Rows rows[2] = {{s->q, q, s->model.nq}, {s->v, v, s->model.nv}};
+  return s->move_rows(false, rows, 2, 1, s->f64, "readback states") ? 0 : 1;
 }
 // phz_readback_states through the library's static per-GPU scratch array
 // instead of the sim's staging buffer: no device allocation on any call.
@@ -2446,8 +2563,8 @@ int phz_readback_states_noalloc(phz_sim* s, double* q, double* v) {
   for (int k = 0; k < 2; k++) {
     if (!parts[k].second || widths[k] <= 0 || s->nworld == 0) continue;
     const size_t bytes = (size_t)s->nworld * widths[k] * sizeof(double);
-    if (!s->hip_ok(phz_io_unpack(parts[k].first, (double*)scr, s->nworld, widths[k], s->stride, s->f64 ? 1 : 0,
-                                 s->stream), "readback_states_noalloc: unpack") ||
+    const PhzRowParts p{{const_cast<void*>(parts[k].first)}, {scr}, {widths[k]}, 1, 0, s->nworld, s->stride};
+    if (!s->hip_ok(phz_io_rows_out(&p, s->f64, 1, s->stream), "readback_states_noalloc: unpack") ||
         !s->hip_ok(hipMemcpyAsync(parts[k].second, scr, bytes, hipMemcpyDeviceToHost, s->stream),
                    "readback_states_noalloc: copy") ||
         !s->hip_ok(hipStreamSynchronize(s->stream), "readback_states_noalloc: sync"))
@@ -2711,15 +2828,10 @@ int phz_readback_policy_history(phz_sim* s, uint32_t start, uint32_t end, double
     return s->fail(fmt("policy history range %u..%u outside 0..%d", start, end, s->pol.history));
   if (!s->has_device()) return s->fail("host-only sim has no device buffers");
   if (!set_device(s)) return 1;
-  const size_t W = (size_t)s->nworld;
-  for (uint32_t k = start; k < end; k++) {
-    if (obs && !s->download_rows(s->obs_row(k), obs + (k - start) * W * s->pol.n_in, s->pol.n_in, "readback obs", 0))
-      return 1;
-    if (out && !s->download_rows(s->out_row(k), out + (k - start) * W * (s->pol.n_out + 1), s->pol.n_out + 1,
-                                 "readback actions", 0))
-      return 1;
-  }
-  return 0;
+  const size_t step = (size_t)s->stride * sizeof(float);
+  const phz_sim::Rows rows[2] = {{s->obs_row(start), obs, s->pol.n_in, s->pol.n_in * step},
+                                 {s->out_row(start), out, s->pol.n_out + 1, (s->pol.n_out + 1) * step}};
+  return s->move_rows(false, rows, 2, (int)(end - start), false, "readback policy history") ? 0 : 1;
 }
 
 int phz_readback_targets(phz_sim* s, double* rows) {
@@ -2768,15 +2880,11 @@ int phz_readback_state_history(phz_sim* s, uint32_t start, uint32_t end, double*
     return s->fail(fmt("history range %u..%u outside 0..%d", start, end, s->hist_slots));
   if (!s->has_device()) return s->fail("host-only sim has no device buffers");
   if (!set_device(s)) return 1;
-  const size_t W = (size_t)s->nworld, E = s->esize(), S = s->stride;
+  const size_t step = (size_t)s->stride * s->esize();
   const int nq = s->model.nq, nv = s->model.nv;
-  for (uint32_t k = start; k < end; k++) {
-    if (q && !s->download_rows((char*)s->hq + k * nq * S * E, q + (k - start) * W * nq, nq, "readback history q"))
-      return 1;
-    if (v && !s->download_rows((char*)s->hv + k * nv * S * E, v + (k - start) * W * nv, nv, "readback history v"))
-      return 1;
-  }
-  return 0;
+  const phz_sim::Rows rows[2] = {{s->hist_row(s->hq, start, nq), q, nq, nq * step},
+                                 {s->hist_row(s->hv, start, nv), v, nv, nv * step}};
+  return s->move_rows(false, rows, 2, (int)(end - start), s->f64, "readback state history") ? 0 : 1;
 }
 
 int phz_rollout(phz_sim* s, uint32_t first_step, uint32_t n_control, uint32_t control_every, int record_states) {

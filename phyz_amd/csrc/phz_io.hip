@@ -3,29 +3,72 @@
 // The C ABI hands over world-major f64 rows (the reference wire layout,
 // crates/phyz-gpu/src/layout.rs:327-373); the step kernel keeps state as
 // structure-of-arrays [j][stride] in the sim's precision so that lane-per-world
-// loads and stores coalesce. These kernels convert between the two on device,
-// so a host upload or readback is one contiguous copy plus one launch.
+// loads and stores coalesce. These kernels move rows between the two layouts.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
 #include <mutex>
 
+constexpr int kPhzRowParts = 3;
+struct PhzRowParts {  // must match phz_host.cpp
+  void* soa[kPhzRowParts];
+  void* rows[kPhzRowParts];
+  int width[kPhzRowParts];
+  int parts, first, count, stride;
+};
+
 namespace {
 
-// dst[j * stride + w] = (T) src[w * width + j]
-template <class T>
-__global__ void pack_rows(const double* __restrict__ src, T* __restrict__ dst, int nworld, int width, int stride) {
-  const int w = blockIdx.x * blockDim.x + threadIdx.x;
-  if (w >= nworld) return;
-  for (int j = 0; j < width; j++) dst[(size_t)j * stride + w] = (T)src[(size_t)w * width + j];
+// World-major rows against structure-of-arrays columns, a tile of 64 worlds x
+// 64 columns through LDS so that both sides are read and written in whole
+// lines; one grid row per part, so q, v and ctrl are one launch. The rows are
+// pinned host memory (RowsArgs in phz_host.cpp), which the kernels access over
+// PCIe themselves: no device staging, no copy command, half the bytes where
+// the sim is f32. Bound by PCIe in large launches and by the launch itself in
+// small ones. The lane-per-world form read and wrote rows 8 bytes a lane, a
+// row's pitch apart, in f64; calls before and after are with move_rows in
+// phz_host.cpp.
+constexpr int kTile = 64;
+
+// rows[w][c] = (R) soa[c][first + w]
+template <class T, class R> __global__ void __launch_bounds__(256) rows_out(PhzRowParts p) {
+  __shared__ T tile[kTile][kTile + 1];
+  const int width = p.width[blockIdx.y], w0 = blockIdx.x * kTile, nw = min(kTile, p.count - w0);
+  const T* soa = (const T*)p.soa[blockIdx.y] + p.first + w0;
+  R* rows = (R*)p.rows[blockIdx.y] + (size_t)w0 * width;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  for (int c0 = 0; c0 < width; c0 += kTile) {
+    const int nc = min(kTile, width - c0);
+    if (lane < nw)
+      for (int c = wave; c < nc; c += 4) tile[lane][c] = soa[(size_t)(c0 + c) * p.stride + lane];
+    __syncthreads();
+    for (int k = threadIdx.x; k < nw * nc; k += 256) {
+      const int w = k / nc, c = k - w * nc;
+      rows[(size_t)w * width + c0 + c] = (R)tile[w][c];
+    }
+    __syncthreads();
+  }
 }
 
-// dst[w * width + j] = (double) src[j * stride + w]
-template <class T>
-__global__ void unpack_rows(const T* __restrict__ src, double* __restrict__ dst, int nworld, int width, int stride) {
-  const int w = blockIdx.x * blockDim.x + threadIdx.x;
-  if (w >= nworld) return;
-  for (int j = 0; j < width; j++) dst[(size_t)w * width + j] = (double)src[(size_t)j * stride + w];
+// soa[c][first + w] = rows[w][c]
+template <class T> __global__ void __launch_bounds__(256) rows_in(PhzRowParts p) {
+  __shared__ T tile[kTile][kTile + 1];
+  const int width = p.width[blockIdx.y], w0 = blockIdx.x * kTile, nw = min(kTile, p.count - w0);
+  T* soa = (T*)p.soa[blockIdx.y] + p.first + w0;
+  const T* rows = (const T*)p.rows[blockIdx.y] + (size_t)w0 * width;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  for (int c0 = 0; c0 < width; c0 += kTile) {
+    const int nc = min(kTile, width - c0);
+#pragma unroll 4
+    for (int k = threadIdx.x; k < nw * nc; k += 256) {
+      const int w = k / nc, c = k - w * nc;
+      tile[w][c] = rows[(size_t)w * width + c0 + c];
+    }
+    __syncthreads();
+    if (lane < nw)
+      for (int c = wave; c < nc; c += 4) soa[(size_t)(c0 + c) * p.stride + lane] = tile[lane][c];
+    __syncthreads();
+  }
 }
 
 template <class T> __global__ void fill_zero(T* __restrict__ dst, size_t n) {
@@ -76,17 +119,22 @@ static __device__ __align__(256) double scratch[kScratchBytes / sizeof(double)];
 
 extern "C" {
 
-hipError_t phz_io_pack(const double* src, void* dst, int nworld, int width, int stride, int f64, hipStream_t s) {
-  if (nworld <= 0 || width <= 0) return hipSuccess;
-  if (f64) hipLaunchKernelGGL(pack_rows<double>, dim3(blocks(nworld)), dim3(kBlock), 0, s, src, (double*)dst, nworld, width, stride);
-  else hipLaunchKernelGGL(pack_rows<float>, dim3(blocks(nworld)), dim3(kBlock), 0, s, src, (float*)dst, nworld, width, stride);
+// soa_f64, rows_f64: the element types; rows of a f32 array may be f64.
+hipError_t phz_io_rows_out(const PhzRowParts* p, int soa_f64, int rows_f64, hipStream_t s) {
+  if (p->count <= 0 || p->parts <= 0) return hipSuccess;
+  const dim3 grid((p->count + kTile - 1) / kTile, p->parts), block(256);
+  if (soa_f64 && rows_f64) hipLaunchKernelGGL(HIP_KERNEL_NAME(rows_out<double, double>), grid, block, 0, s, *p);
+  else if (soa_f64) return hipErrorInvalidValue;
+  else if (rows_f64) hipLaunchKernelGGL(HIP_KERNEL_NAME(rows_out<float, double>), grid, block, 0, s, *p);
+  else hipLaunchKernelGGL(HIP_KERNEL_NAME(rows_out<float, float>), grid, block, 0, s, *p);
   return hipGetLastError();
 }
 
-hipError_t phz_io_unpack(const void* src, double* dst, int nworld, int width, int stride, int f64, hipStream_t s) {
-  if (nworld <= 0 || width <= 0) return hipSuccess;
-  if (f64) hipLaunchKernelGGL(unpack_rows<double>, dim3(blocks(nworld)), dim3(kBlock), 0, s, (const double*)src, dst, nworld, width, stride);
-  else hipLaunchKernelGGL(unpack_rows<float>, dim3(blocks(nworld)), dim3(kBlock), 0, s, (const float*)src, dst, nworld, width, stride);
+hipError_t phz_io_rows_in(const PhzRowParts* p, int f64, hipStream_t s) {
+  if (p->count <= 0 || p->parts <= 0) return hipSuccess;
+  const dim3 grid((p->count + kTile - 1) / kTile, p->parts), block(256);
+  if (f64) hipLaunchKernelGGL(rows_in<double>, grid, block, 0, s, *p);
+  else hipLaunchKernelGGL(rows_in<float>, grid, block, 0, s, *p);
   return hipGetLastError();
 }
 

@@ -213,31 +213,31 @@ class BatchSim:
         self._check(self._L.phz_set_controls(self._h, _dp(_rows(ctrl, self.nworld, self.nctrl, "ctrl"))))
 
     def readback_states(self):
-        q = np.zeros((self.nworld, self.nq))
-        v = np.zeros((self.nworld, self.nv))
+        q = np.empty((self.nworld, self.nq))
+        v = np.empty((self.nworld, self.nv))
         self._check(self._L.phz_readback_states(self._h, _dp(q), _dp(v)))
         return q, v
 
     def readback_states_noalloc(self):
         """readback_states through the library's static per-GPU scratch (no
         device allocation); worlds x max(nq, nv) x 8 bytes at most 32 MiB."""
-        q = np.zeros((self.nworld, self.nq))
-        v = np.zeros((self.nworld, self.nv))
+        q = np.empty((self.nworld, self.nq))
+        v = np.empty((self.nworld, self.nv))
         self._check(self._L.phz_readback_states_noalloc(self._h, _dp(q), _dp(v)))
         return q, v
 
     def readback_contacts(self) -> np.ndarray:
-        rows = np.zeros((self.nworld, self.nb, 8))
+        rows = np.empty((self.nworld, self.nb, 8))
         self._check(self._L.phz_readback_contacts(self._h, _dp(rows)))
         return rows
 
     def readback_controls(self) -> np.ndarray:
-        c = np.zeros((self.nworld, self.nctrl))
+        c = np.empty((self.nworld, self.nctrl))
         self._check(self._L.phz_readback_controls(self._h, _dp(c)))
         return c
 
     def readback_qdd(self) -> np.ndarray:
-        a = np.zeros((self.nworld, self.nv))
+        a = np.empty((self.nworld, self.nv))
         self._check(self._L.phz_readback_qdd(self._h, _dp(a)))
         return a
 
@@ -300,7 +300,7 @@ class BatchSim:
 
     def readback_kinematics(self) -> np.ndarray:
         """[nworld][nb][18]: rotation world->body (row-major), origin, omega, v (body frame)."""
-        rows = np.zeros((self.nworld, self.nb, XF_STRIDE))
+        rows = np.empty((self.nworld, self.nb, XF_STRIDE))
         self._check(self._L.phz_readback_kinematics(self._h, _dp(rows)))
         return rows
 
@@ -339,13 +339,13 @@ class BatchSim:
         """(obs [n][nworld][n_in], out [n][nworld][n_out + 1]) for control steps [start, end)."""
         spec = self._policy_spec()
         n = max(int(end) - int(start), 0)
-        obs = np.zeros((n, self.nworld, spec.n_in()))
-        out = np.zeros((n, self.nworld, spec.n_out() + 1))
+        obs = np.empty((n, self.nworld, spec.n_in()))
+        out = np.empty((n, self.nworld, spec.n_out() + 1))
         self._check(self._L.phz_readback_policy_history(self._h, int(start), int(end), _dp(obs), _dp(out)))
         return obs, out
 
     def readback_targets(self) -> np.ndarray:
-        rows = np.zeros((self.nworld, max(self._npd, 1)))
+        rows = np.empty((self.nworld, max(self._npd, 1)))
         self._check(self._L.phz_readback_targets(self._h, _dp(rows)))
         return rows[:, :self._npd]
 
@@ -358,8 +358,8 @@ class BatchSim:
     def readback_state_history(self, start: int, end: int):
         """(q [n][nworld][nq], v [n][nworld][nv]) for history slots [start, end)."""
         n = max(int(end) - int(start), 0)
-        q = np.zeros((n, self.nworld, self.nq))
-        v = np.zeros((n, self.nworld, self.nv))
+        q = np.empty((n, self.nworld, self.nq))
+        v = np.empty((n, self.nworld, self.nv))
         self._check(self._L.phz_readback_state_history(self._h, int(start), int(end), _dp(q), _dp(v)))
         return q, v
 
