@@ -1449,9 +1449,13 @@ struct phz_sim {
   size_t hf_cap = 0;                                                // node capacity of hf_buf
   uint64_t* rng = nullptr;
   // Pinned host memory that state rows pass through, kSlots slots used in turn
-  // (move_rows): at most 4 x 512 KB, or 4 x 64 worlds' rows where those are more.
+  // (move_rows): at most 4 x 512 KB in f32 and 4 x 1 MB in f64, or 4 x 64
+  // worlds' rows where those are more. us a pass with slots of 32, 64, 128 and
+  // 256 K values: f32 env step of 8192 237 (64 K), 200, 207 (256 K), chain
+  // 65536 x 20 494 (64 K), 430, 412 (256 K); f64 hand 16384 x 200 1300 (32 K),
+  // 1030 (64 K), 960 (128 K).
   static constexpr int kSlots = 4;
-  static constexpr size_t kSlotBytes = size_t(512) << 10;
+  static constexpr size_t kSlotValues = size_t(128) << 10;
   char* pin = nullptr;
   size_t pin_slot = 0;
   hipEvent_t pin_ev[kSlots] = {};
@@ -1583,7 +1587,7 @@ struct phz_sim {
     if (np == 0 || W == 0 || groups <= 0) return true;
     // A slot holds whole tiles of 64 worlds, each part from a 256-byte boundary.
     const size_t pad = 256 * kPhzRowParts, tiles = (W + 63) / 64, tile_bytes = 64 * per_world;
-    const size_t fit = std::max<size_t>(1, kSlotBytes > pad ? (kSlotBytes - pad) / tile_bytes : 1);
+    const size_t fit = std::max<size_t>(1, (kSlotValues * E - pad) / tile_bytes);
     const size_t cw = 64 * std::min(tiles, fit), per_group = (W + cw - 1) / cw, chunks = per_group * groups;
     if (!ensure_pin((cw * per_world + pad + 4095) & ~size_t(4095))) return false;
     for (int k = 1; k < np; k++) off[k] = (off[k - 1] + cw * part[k - 1].width * E + 255) & ~size_t(255);
