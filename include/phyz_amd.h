@@ -193,6 +193,12 @@ int phz_kernel_info(phz_sim* sim, int64_t* info);
  * crates/phyz-gpu/cuda/phyz_kernels.cu); it reports this build's launch
  * layout. Works on host-only sims. */
 int phz_lanes_per_world(phz_sim* sim);
+/* Bytes of pinned host memory that the sim holds once a call has moved rows of
+ * `width` values a world, f64 nonzero for double precision (width 0: once
+ * phz_compile has run). Calls that move rows stage them there; the memory is
+ * allocated by phz_compile or the first such call, and again only by a call
+ * with a larger answer here than every one before. Works on host-only sims. */
+uint64_t phz_staging_bytes(phz_sim* sim, uint32_t width, int f64);
 
 /* ── Device-resident control loop (mod.rs:1004-1376; policy_pipeline.rs) ──── */
 

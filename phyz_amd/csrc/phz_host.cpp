@@ -1453,7 +1453,8 @@ struct phz_sim {
   // worlds' rows where those are more. us a pass with slots of 32, 64, 128 and
   // 256 K values: f32 env step of 8192 237 (64 K), 200, 207 (256 K), chain
   // 65536 x 20 494 (64 K), 430, 412 (256 K); f64 hand 16384 x 200 1300 (32 K),
-  // 1030 (64 K), 960 (128 K).
+  // 1030 (64 K), 960 (128 K). Allocated by phz_compile or by the first call
+  // that moves rows, in a size that the sim's other calls share (slot_bytes).
   static constexpr int kSlots = 4;
   static constexpr size_t kSlotValues = size_t(128) << 10;
   char* pin = nullptr;
@@ -1524,6 +1525,32 @@ struct phz_sim {
     if (!hip_ok(hipMalloc(p, std::max<size_t>(bytes, 256)), what)) return false;
     return hip_ok(phz_io_zero(*p, std::max<size_t>(bytes, 256), stream), what);
   }
+  // Worlds of a slot for rows of per_world bytes (whole tiles of 64).
+  static constexpr size_t kPartPad = 256 * kPhzRowParts;  // each part starts at a 256-byte boundary
+  size_t slot_worlds(size_t per_world, size_t elem) const {
+    const size_t tiles = ((size_t)nworld + 63) / 64;
+    return 64 * std::min(tiles, std::max<size_t>(1, (kSlotValues * elem - kPartPad) / (64 * per_world)));
+  }
+  // The slot size of a call that moves per_world bytes a world (0: none yet).
+  // Full slots of different row widths differ by a few pages, and a call that
+  // outgrew the one before waited for the queued span, freed the slots and
+  // pinned them anew in the middle of a pass (the first pass of a fresh sim,
+  // us: f64 chain 65536 x 1000 8770, now 4750; pendulum 96 x 25 421, now 308).
+  // So a call that takes several
+  // slots, or more than half of one, gets the full size, a smaller one a power
+  // of two, and none less than the state and contact rows need.
+  size_t slot_bytes(size_t per_world, size_t elem) const {
+    auto need = [&](size_t bytes, size_t e) {
+      if (bytes == 0 || nworld == 0) return size_t(0);
+      const size_t n = (slot_worlds(bytes, e) * bytes + kPartPad + 4095) & ~size_t(4095), cap = kSlotValues * e;
+      if (n > cap / 2) return std::max(n, cap);
+      size_t p = 4096;
+      while (p < n) p *= 2;
+      return p;
+    };
+    const size_t e = esize(), state = (size_t)(model.nq + model.nv + nctrl()) * e;
+    return std::max({need(per_world, elem), need(state, e), feat.contact ? need((size_t)model.nb * 8 * e, e) : 0});
+  }
   bool ensure_pin(size_t slot) {
     for (auto& e : pin_ev)
       if (!e && !hip_ok(hipEventCreateWithFlags(&e, hipEventDisableTiming), "staging event")) return false;
@@ -1585,11 +1612,8 @@ struct phz_sim {
         per_world += rows[k].width * E;
       }
     if (np == 0 || W == 0 || groups <= 0) return true;
-    // A slot holds whole tiles of 64 worlds, each part from a 256-byte boundary.
-    const size_t pad = 256 * kPhzRowParts, tiles = (W + 63) / 64, tile_bytes = 64 * per_world;
-    const size_t fit = std::max<size_t>(1, (kSlotValues * E - pad) / tile_bytes);
-    const size_t cw = 64 * std::min(tiles, fit), per_group = (W + cw - 1) / cw, chunks = per_group * groups;
-    if (!ensure_pin((cw * per_world + pad + 4095) & ~size_t(4095))) return false;
+    const size_t cw = slot_worlds(per_world, E), per_group = (W + cw - 1) / cw, chunks = per_group * groups;
+    if (!ensure_pin(slot_bytes(per_world, E))) return false;
     for (int k = 1; k < np; k++) off[k] = (off[k - 1] + cw * part[k - 1].width * E + 255) & ~size_t(255);
     auto launch = [&](size_t i) {
       const size_t g = i / per_group, first = i % per_group * cw, slot = i % kSlots;
@@ -2618,6 +2642,9 @@ int phz_collidable_bodies(const phz_sim* s) { return s && s->feat.contact ? s->f
 int phz_compile(phz_sim* s) {
   if (!s) return 1;
   if (!s->compile()) return 1;
+  // The slots' memory is not the first pass's to wait for (where it cannot be
+  // had, the call that moves rows says so).
+  if (s->has_device() && s->nworld > 0 && set_device(s)) (void)s->ensure_pin(s->slot_bytes(0, s->esize()));
   if ((s->kin_on || s->policy_on) && !s->ensure_ctl(false, false)) return 1;
   if (s->policy_on && !s->ensure_ctl(true, false)) return 1;
   return 0;
@@ -2652,6 +2679,12 @@ int phz_lanes_per_world(phz_sim* s) {
   if (!s) return -1;
   if (!s->compile()) return -1;
   return s->lanes;
+}
+
+uint64_t phz_staging_bytes(phz_sim* s, uint32_t width, int f64) {
+  if (!s) return 0;
+  const size_t e = f64 ? 8 : 4;
+  return phz_sim::kSlots * s->slot_bytes(width * e, e);
 }
 
 int phz_kernel_info(phz_sim* s, int64_t* info) {

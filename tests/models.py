@@ -107,6 +107,21 @@ def random_tree(seed, njoints=8, with_free_root=True):
     return b.build()
 
 
+def legged(legs, links):
+    """A free sphere torso on `legs` legs of `links` hinged capsules each."""
+    b = ModelBuilder().gravity([0, 0, -G]).dt(0.002).add_free_body(
+        "torso", -1, SpatialTransform.identity(), iso(5.0, 0.1), Geometry.sphere(0.15))
+    for i in range(legs):
+        a, parent = 2 * math.pi * i / legs, 0
+        for j in range(links):
+            at = [0.2 * math.cos(a), 0.2 * math.sin(a), 0.0] if j == 0 else [0.0, 0.0, -0.2]
+            b.add_body(f"leg{i}_{j}", parent, Joint(REVOLUTE, SpatialTransform.from_translation(at), np.array([0.0, 1.0, 0.0])),
+                       SpatialInertia.new(0.5, [0, 0, -0.1], np.eye(3) * 0.005),
+                       Geometry.capsule(0.03, 0.2, SpatialTransform.from_translation([0, 0, -0.1])))
+            parent = 1 + i * links + j
+    return b.build()
+
+
 def trunk_and_two_feet():
     """Free trunk with two hinged feet, offset centres of mass (cuda_vs_cpu.rs:1418-1443)."""
     def off(m, c):
