@@ -229,6 +229,7 @@ struct Plan {
   int mode = 0;
   std::vector<int> trunk;                // topological order
   std::vector<std::vector<int>> groups;  // bodies owned by each wave, topological order
+  double speedup = 0;  // small floating trees: one lane's modelled step length over this plan's
 };
 
 Plan plan_partition(const ModelD& m, const Features& f) {
@@ -309,15 +310,11 @@ Plan plan_partition(const ModelD& m, const Features& f) {
   }
   const bool forced = want == "1" || want == "2";
   if (parts.size() < 2) return lane_per_world();
-  // Trees of fewer than 14 bodies (the ants) are partitioned in f32 launches of
-  // up to three workgroups per CU, where the waves per world group fill SIMDs
-  // that a lane per world leaves idle or lightly loaded; their kernels hold at
-  // most 256 registers, so workgroups share SIMDs and none waits for a further
-  // round (phz_sim::compile takes the lane plan back where one does not).
-  // Measured, us per 100-step launch, lane per world / 4 waves: ant 64 worlds
-  // 447 / 259, 16384 465 / 278, 32768 472 / 362, 49152 485 / 446, 65536 502 /
-  // 637; with PD servos 427 / 230 to 464 / 423 at 49152; MJCF ant 807 / 325,
-  // 826 / 357, 836 / 493, 865 / 779, 882 / 930. f64 keeps one lane per world.
+  // Trees of fewer than 14 bodies are partitioned in f32 launches of up to
+  // three workgroups per CU, where the waves per world group fill SIMDs that a
+  // lane per world leaves idle or lightly loaded, as far as phz_sim::
+  // small_tree_pays finds it worth while from the compiled kernel's registers.
+  // f64 keeps one lane per world.
   const bool small_tree = mode == 2 && nb < 14 && !f.f64;
   if (mode == 2 && !forced && nb < 14 && (f.f64 || f.lane_small_tree || f.wgs > 3 * std::max(f.cus, 1)))
     return lane_per_world();
@@ -364,8 +361,8 @@ Plan plan_partition(const ModelD& m, const Features& f) {
   auto cost = [&](const std::vector<double>& load) {
     const int ng = (int)load.size(), cus = std::max(f.cus, 1);
     const long per_cu = std::max(1, (f.wgs + cus - 1) / cus);
-    const long conc = (ng <= 4 ? 4 / ng : 1) * (small_tree ? 4 : 1);
-    const long rounds = (per_cu + conc - 1) / conc;
+    const long conc = ng <= 4 ? 4 / ng : 1;
+    const long rounds = small_tree ? 1 : (per_cu + conc - 1) / conc;  // small trees' waves share SIMDs
     double simd[4] = {0, 0, 0, 0};
     for (int k = 0; k < ng; k++) simd[k % 4] += load[k] + pass1 + (k == 0 ? tcontact : 0.0);
     return (double)rounds * (*std::max_element(simd, simd + 4) + serial);
@@ -471,6 +468,16 @@ Plan plan_partition(const ModelD& m, const Features& f) {
     }
   }
   pl.mode = mode;
+  if (small_tree) {
+    std::vector<double> load;
+    double all = twt + tcontact;
+    for (auto& p : parts) {
+      load.push_back(0);
+      for (int i : p) load.back() += weight(i);
+      all += load.back();
+    }
+    pl.speedup = all / cost(load);
+  }
   for (int i = 0; i < nb; i++) if (trunk[i]) pl.trunk.push_back(i);
   for (auto& p : parts) {
     std::sort(p.begin(), p.end());
@@ -1672,11 +1679,11 @@ struct phz_sim {
     int ng = 1;
     feat.lane_small_tree = false;
     std::string src = gen_source(model, feat, f64, &ng, &lanes);
-    if (ng > 1 && model.nb < 14 && !f64 && feat.wgs > feat.cus) {
-      // The plan of a small tree counts on two waves per SIMD (plan_partition).
+    const double speedup = plan_partition(model, feat).speedup;
+    if (speedup > 0 && feat.wgs > feat.cus) {
       std::string e2;
       const auto co = compile_source(src, Build::Reassoc, e2);
-      if (co && remark_value(co->log, "VGPRs:") + std::max<int64_t>(remark_value(co->log, "AGPRs:"), 0) > 256) {
+      if (co && !small_tree_pays(co->log, ng, speedup)) {
         feat.lane_small_tree = true;
         src = gen_source(model, feat, f64, &ng, &lanes);
       }
@@ -1726,6 +1733,35 @@ struct phz_sim {
     }
     if (!code) { err = e; return false; }
     return true;
+  }
+  // Whether a small tree's partitioned kernel (compiled to `log`, ng waves per
+  // world group) beats one lane per world in a launch of more than one
+  // workgroup per CU. What its workgroups cost, as multiples of one per CU:
+  // the second 1.0-1.5, less than every plan gains; the third 1.4-1.6 where
+  // the registers let it in and 2.0-2.2 where it waits for a wave slot. The
+  // modelled speedup (plan_partition) is 1.0-1.4 times the measured one, more
+  // for the plans of four waves. us per 100-step launch, one lane / partition,
+  // at 64, 32768 and 49152 worlds (one, two and three workgroups per CU):
+  //   4 waves, registers for three: ant (model 2.40) 445 / 261, 477 / 363, 483 / 440; with
+  //   PD servos 426 / 233, 457 / 332, 460 / 413
+  //   4 waves, for two: MJCF ant (2.42) 803 / 324, 832 / 505, 840 / 755;
+  //   four legs of three links (2.73) 758 / 293, 786 / 473, 799 / 706; six legs
+  //   of two (2.41) 749 / 340, 775 / 517, 808 / 778; five legs of two (2.06)
+  //   591 / 334, 627 / 467, 632 / 739; nine bodies of mixed
+  //   joints (1.31) 795 / 567, 820 / 650, 841 / 1167
+  //   2 waves, for four: two legs of two (1.42) 294 / 217, 311 / 311, 322 /
+  //   318; three legs of two (1.35) 387 / 312, 411 / 395, 423 / 441; two legs
+  //   of three (1.53) 393 / 269, 417 / 398, 429 / 433; three free bodies
+  //   (1.71) 471 / 277, 495 / 392, 502 / 400
+  //   2 waves, for two: three legs of three (1.39) 552 / 420, 579 / 459, 591 /
+  //   879; two legs of six (1.71) 768 / 435, 800 / 490, 818 / 926
+  // Four per CU: ant 501 / 623, MJCF ant 877 / 945 (plan_partition stops at three).
+  bool small_tree_pays(const std::string& log, int ng, double speedup) const {
+    const int64_t regs = remark_value(log, "VGPRs:") + std::max<int64_t>(remark_value(log, "AGPRs:"), 0);
+    const long resident = 4 * (512 / std::max<long>((regs + 7) & ~7L, 8)) / ng;
+    const long cus = std::max(feat.cus, 1), per_cu = (feat.wgs + cus - 1) / cus;
+    if (resident < 2) return false;
+    return per_cu <= 2 || speedup > (resident >= per_cu ? 1.55 : 2.3);
   }
   // Whether the one-wave-per-world-group kernel compiled to `log` gets a
   // second build for two resident waves per SIMD: it holds more than 256
