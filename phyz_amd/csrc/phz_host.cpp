@@ -1880,23 +1880,39 @@ struct phz_sim {
   float* out_row(uint32_t step) const { return out_hist + (size_t)step * (pol.n_out + 1) * stride; }
 
   // The workgroup-per-tile policy kernel's tile for a launch of this size, in
-  // 16-world columns; 0: one wave per tile. It runs up to four columns per CU,
-  // as 16-world tiles (4 waves) up to one per CU, beyond that and for wide
-  // nets as 32-world tiles (8 waves), which read the weights half as often.
-  // us per launch, one wave per tile / 16-world / 32-world tiles:
-  //   29 inputs, hidden 256, 8 actions: 64 worlds 40 / 15.8 / 18.0, 4096 41 /
-  //   17.9 / 19.1, 8192 42 / 23.0 / 20.6, 16384 44 / 38.4 / 29.2, 32768 49 /
-  //   67 / 51.5; hidden 64: 4096 26 / 12.2 / 13.8, 16384 27 / 17.6 / 18.0,
-  //   24576 28 / 24.6 / 28.8;
-  //   128, 256, 32: 4096 79 / 36.4 / 38.0, 8192 81 / 46.2 / 40.0, 16384 86 /
-  //   85.7 / 70.2.
+  // 16-world columns; 0: one wave per tile. Up to one column per CU a 16-world
+  // tile (4 waves), up to two a 32-world tile (8 waves, which read the weights
+  // half as often); beyond, nets of up to 128 hidden neurons (one pair of
+  // blocks per wave of 4) take the 16-world tile, whose small workgroups share
+  // a CU, up to six columns per CU (five at 32, whose one-wave form is as
+  // short), and wider ones the 32-world tile up to four (at five 29-160-8
+  // would still gain, 29-200-8 and the wider ones lose: 35.1 40.5 37.8).
+  // us per launch, one wave per tile / 16-world / 32-world tiles, at 64, 4096,
+  // 8192, 12288, 16384, 20480 and 24576 worlds (256 columns are 4096):
+  //   29-32-8    20.7 10.9 12.3, 20.7 11.6 13.0, 21.0 13.4 13.4, 21.2 13.8 15.9,
+  //              21.4 15.8 16.3, 22.6 21.5 26.1, 22.8 23.3 26.6
+  //   29-64-8    25.2 11.4 12.9, 25.2 12.2 13.6, 25.6 14.4 14.2, 25.9 15.1 17.5,
+  //              26.2 17.6 18.1, 27.3 19.7 26.0, 27.7 24.7 29.0 (32768 28.4 28.3 30.8)
+  //   29-128-8   36.6 12.2 14.5, 36.8 13.1 15.2, 37.2 16.1 16.1, 37.7 17.5 20.8,
+  //              38.1 20.7 21.7, 39.4 23.3 30.1, 39.9 28.4 34.8
+  //   29-160-8   37.3 14.6 15.8, 37.0 15.6 16.8, 37.6 19.6 17.7, 38.2 22.4 22.5,
+  //              39.5 31.6 23.4, 40.1 35.7 33.1, 40.5 40.2 38.0
+  //   29-256-8   37.5 16.0 17.9, 38.6 17.8 19.1, 39.7 23.2 20.7, 40.9 27.9 27.6,
+  //              41.9 38.7 29.1, 43.3 44.4 40.4, 44.2 50.5 42.2 (32768 47.0 65.8 52.1)
+  //   60-48-20   40.1 17.9 19.9, 40.2 18.9 20.9, 40.7 22.8 21.7, 41.2 23.9 26.6,
+  //              41.7 27.4 27.8, 43.5 37.9 40.7, 44.0 39.0 41.7
+  //   128-64-32  73.2 29.2 31.5, 73.9 30.3 32.9, 74.9 36.4 34.2, 75.9 39.1 56.3,
+  //              76.6 56.3 59.0, 80.0 62.6 80.6, 81.0 70.2 83.0 (32768 81.9 92.6 106.7)
+  //   128-256-32 77.3 33.1 35.1, 79.4 36.5 38.0, 81.2 46.8 40.2, 83.8 72.2 67.5,
+  //              85.7 85.4 70.6, 87.5 107.8 97.5, 89.0 123.1 100.6
   // PHZ_POLICY_TEAM=0|1|2 forces the form (tests, tuning).
   int team_columns() const {
     if (!pol.split) return 0;
     if (const char* e = std::getenv("PHZ_POLICY_TEAM")) return std::max(0, std::min(2, std::atoi(e)));
     const long columns = ((long)nworld + 15) / 16, cus = std::max(feat.cus, 1);
-    if (columns > 4 * cus) return 0;
-    return columns > cus || pol.n_in + pol.n_out > 64 ? 2 : 1;
+    const bool wide = pol.nhb() > 8;
+    if (columns > cus * (wide ? 4 : pol.nhb() > 2 ? 6 : 5)) return 0;
+    return columns > cus && (wide || columns <= 2 * cus) ? 2 : 1;
   }
   // Compile (and with `load`, load) the FK/observation or the policy kernel
   // for the current configuration epoch.
