@@ -354,12 +354,16 @@ __device__ __forceinline__ void mfma_layer(const f32x4* __restrict__ w, int lane
 // ── layers 2 and 3 in three bf16 pieces ──
 // An f32 is the exact sum of three bf16 values, each the rounding of what the
 // ones before it left (8 significant bits each, signed remainders):
-// x = h + m + l. A product then needs the six partial products of relative
-// size above 2^-24: hh, hm, mh, hl, lh, mm; the three dropped ones (ml, lm, ll)
-// are below 2^-26 of it. bf16 products are exact in f32 and the MFMA sums 32
-// of them with one rounding where the f32 MFMA rounds per 4, so the layer's
-// error against 64 bits is no larger than the f32 MFMA's (measured in
-// tests/test_gpu_policy_split.py). Six 16x16x32 bf16 MFMAs (16 cycles each)
+// x = h + m + l with |m| <= 2^-8 |x|, |l| <= 2^-17 |x|. A product takes the
+// six partial products hh, hm, mh, hl, lh, mm; the dropped ml and lm are up to
+// 2^-25 of it each (ll 2^-34), half a unit in the last place of an f32 product
+// together where both operands' pieces are at their largest with one sign. In
+// return bf16 products are exact in f32 and the MFMA sums 32 of them with one
+// rounding where the f32 MFMA rounds per 4: six roundings per 32 inputs
+// against eight. That the layer's error against 64 bits is no larger is
+// measured (tests/test_gpu_policy_split.py): 0.69-0.99 of the f32 MFMA's over
+// random weights, 0.75-0.93 with every weight at 2^-8 and 2^-17 pieces of one
+// sign, 0.05-1.01 with equal activations of that kind too. Six 16x16x32 bf16 MFMAs (16 cycles each)
 // replace eight 16x16x4 f32 ones (32 cycles each) per 32 inputs: 96 against
 // 256 cycles of matrix core, for 5.5 more VALU instructions per activation.
 // 29-256-256-8, us per launch (f32, split): 56, 41 at 4096 worlds, 122, 79 at
@@ -369,8 +373,9 @@ __device__ __forceinline__ void mfma_layer(const f32x4* __restrict__ w, int lane
 // 34000 cycles of MFMA per wave, which the two waves of a SIMD overlap by
 // little.
 // Taken where every weight of the two layers is zero or of magnitude in
-// [2^-100, 2^100] (the host checks on upload), so that no piece overflows or
-// is subnormal; their inputs are tanh values. The first layer stays f32: its
+// [2^-100, 2^100] (the host checks on upload), so that none of its pieces
+// overflows or is subnormal. Their inputs are tanh values, at most 1; of one
+// below 2^-103 the bits under 2^-126 may be lost. The first layer stays f32: its
 // inputs are the caller's observations, of any range.
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x8 __attribute__((ext_vector_type(8)));

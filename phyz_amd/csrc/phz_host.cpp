@@ -1171,7 +1171,7 @@ float bf16_value(uint16_t b) {
 // hold every weight with no piece infinite or subnormal (zero, or a magnitude
 // in [2^-100, 2^100]), and a layer has at least 32 inputs, from where its
 // error against 64 bits is below the f32 MFMA's (ratio of the two over weight
-// scales 0.05 to 3: 0.73-0.96 at widths 32 to 256, 0.77-1.03 at 24, 0.79-1.18
+// scales 0.05 to 3: 0.69-0.99 at widths 32 to 256, 0.77-1.03 at 24, 0.79-1.18
 // at 16, where nothing is gained in time either: 20.0 against 20.1 us).
 constexpr int kSplitMinHidden = 32;
 bool policy_splits(const PolicyD& p, const double* w) {
