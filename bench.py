@@ -71,6 +71,7 @@ sys.path.insert(0, ROOT)
 
 METRIC = "world-steps/sec (ABA+contact+integrate) on 1 MI355X; % of HBM/FP64 roofline"
 PEAK_TFLOPS = {"f64": 78.6, "f32": 157.3}
+PEAK_BF16_MFMA = 2516.6  # dense: 16384 FLOP in 16 cycles on 1024 SIMDs at 2.4 GHz
 HBM_PEAK_GBS = 8000.0
 FLOPS_JSON = os.path.join(ROOT, "tests", "golden", "flops_per_world_step.json")
 TRAFFIC_JSON = os.path.join(ROOT, "profiles", "hbm_traffic.json")
@@ -412,6 +413,15 @@ def run_world_sweep(idx=2, sizes=SWEEP_WORLDS, precs=("f32", "f64"), steps=100, 
     return out
 
 
+def policy_peak_tflops(n_in: int, hidden: int, n_out: int) -> float:
+    """The rate, in the MLP's own FLOP, at which the matrix cores could run the
+    policy kernel's layers: layer 1 on the f32 instruction (157.3 TFLOP/s),
+    layers 2 and 3 as six bf16 products each from 32 hidden neurons on."""
+    first, rest = n_in * hidden, hidden * (hidden + n_out)
+    t = first / PEAK_TFLOPS["f32"] + (6 * rest / PEAK_BF16_MFMA if hidden >= 32 else rest / PEAK_TFLOPS["f32"])
+    return (first + rest) / t
+
+
 def run_control_loop(prec: str, reps: int, with_cpu: bool):
     """The ant driven by the on-device policy (phyz_amd.workloads.control_loop):
     a rollout of n_control control steps, each FK + observation, the MLP policy,
@@ -440,6 +450,8 @@ def run_control_loop(prec: str, reps: int, with_cpu: bool):
     m = cl.base.model
     obs_bytes = n * 4 * ((m.nq + m.nv) + 18 * m.nbodies + cl.spec.n_in())
     pol_flops = cl.flops_per_world() * n
+    pol_rate = pol_flops / (t_pol / 1e3) / 1e12
+    pol_peak = policy_peak_tflops(cl.spec.n_in(), cl.spec.hidden, cl.spec.n_out())
     out = {
         "workload": cl.name, "nworld": n, "n_control": nc, "control_every": every, "dtype": prec,
         "mlp": [cl.spec.n_in(), cl.spec.hidden, cl.spec.hidden, cl.spec.n_out()],
@@ -447,8 +459,9 @@ def run_control_loop(prec: str, reps: int, with_cpu: bool):
         "world_steps_per_s": round(n * nc * every / (t_roll / 1e3), 1),
         "control_steps_per_s": round(n * nc / (t_roll / 1e3), 1),
         "physics_only_ms": round(t_phys, 4),
-        "policy_roofline": {"bound": "mfma", "achieved": round(pol_flops / (t_pol / 1e3) / 1e12, 3), "peak": 157.3,
-                            "unit": "TFLOP/s", "frac": round(pol_flops / (t_pol / 1e3) / 1e12 / 157.3, 4),
+        "policy_roofline": {"bound": "mfma", "achieved": round(pol_rate, 3), "peak": round(pol_peak, 1),
+                            "unit": "TFLOP/s", "frac": round(pol_rate / pol_peak, 4),
+                            "peak_of": "layer 1 in f32, layers 2 and 3 as six bf16 products each",
                             "launch_ms": round(t_pol, 5), "flops_per_world": cl.flops_per_world(),
                             "kernel": sim.control_kernel_info("policy")},
         "obs_roofline": {"bound": "hbm", "achieved": round(obs_bytes / (t_obs / 1e3) / 1e9, 1), "peak": HBM_PEAK_GBS,
