@@ -55,6 +55,9 @@ the reference's timing shape (a million samples, actor 55-64-64-22, critic
 whole updates, the tile kernel's roofline from kernel-stamped hipEvents, and, with the CPU
 leg, the f64 CPU update on 128 minibatches plus the device's update of that
 sample against it.
+
+The line on stdout holds the headline in full and the other measurements'
+figures; --details FILE writes all of them in full.
 """
 from __future__ import annotations
 
@@ -686,8 +689,48 @@ def config_of(w, r):
     return c
 
 
+def _brief(e):
+    """A measurement's figures without its kernel, configuration and samples."""
+    out = {k: e[k] for k in ("value", "ms_per_step", "finite_worlds", "gpu_over_cpu", "seconds_per_update") if k in e}
+    if e.get("roofline"):
+        out.update({k: e["roofline"][k] for k in ("achieved", "frac", "launch_ms")})
+    if e.get("cpu_baseline"):
+        out["cpu"] = e["cpu_baseline"]["value"]
+    if "pass" in (e.get("parity") or {}):
+        out["parity"] = "pass" if e["parity"]["pass"] else "FAIL"
+    if "io" in e:
+        out["load_span_readback_ms"] = e["io"]["load_span_readback_ms"]
+    return out
+
+
+def brief_line(line):
+    """The line that goes to stdout: the headline in full, every other
+    measurement in its figures, so that it stays a few thousand characters."""
+    out = dict(line)
+    if "configs" in out:
+        out["configs"] = {name: {pr: _brief(e[pr]) for pr in ("f32", "f64") if pr in e} for name, e in out["configs"].items()}
+    for key in ("terrain_impulse", "ppo_update"):
+        if key in out:
+            out[key] = _brief(out[key])
+    if "mjcf" in out:
+        out["mjcf"] = {name: _brief(e) for name, e in out["mjcf"].items()}
+    if "world_sweep" in out:
+        sweep = {}
+        for e in out["world_sweep"]:
+            sweep.setdefault(e["dtype"], {})[str(e["nworld"])] = float(f"{e['world_steps_per_s_event']:.4g}")
+        out["world_sweep"] = sweep
+    if "control_loop" in out:
+        e = out["control_loop"]
+        out["control_loop"] = {"world_steps_per_s": e["world_steps_per_s"], "rollout_ms": e["rollout_ms"]["median"],
+                               "physics_only_ms": e["physics_only_ms"],
+                               **{k: {f: e[k][f] for f in ("achieved", "peak", "frac", "launch_ms")}
+                                  for k in ("policy_roofline", "obs_roofline")}}
+    return out
+
+
 def main():
     ap = argparse.ArgumentParser()
+    ap.add_argument("--details", metavar="FILE", help="also write every measurement in full to FILE, as JSON")
     ap.add_argument("--gpus", type=int, default=1)
     ap.add_argument("--steps", type=int, default=None,
                     help="timed steps of the headline workload (default: its rollout length)")
@@ -832,7 +875,10 @@ def main():
         line["control_loop"] = run_control_loop("f32", min(args.reps, 5), with_cpu)
     if not args.no_ppo:
         line["ppo_update"] = run_ppo_update(min(args.reps, 5), with_cpu)
-    print(json.dumps(line), flush=True)
+    if args.details:
+        with open(args.details, "w") as f:
+            json.dump(line, f)
+    print(json.dumps(brief_line(line)), flush=True)
 
 
 if __name__ == "__main__":
