@@ -363,15 +363,16 @@ __device__ __forceinline__ void mfma_layer(const f32x4* __restrict__ w, int lane
 // against eight. That the layer's error against 64 bits is no larger is
 // measured (tests/test_gpu_policy_split.py): 0.69-0.99 of the f32 MFMA's over
 // random weights, 0.75-0.93 with every weight at 2^-8 and 2^-17 pieces of one
-// sign, 0.05-1.01 with equal activations of that kind too. Six 16x16x32 bf16 MFMAs (16 cycles each)
-// replace eight 16x16x4 f32 ones (32 cycles each) per 32 inputs: 96 against
-// 256 cycles of matrix core, for 5.5 more VALU instructions per activation.
-// 29-256-256-8, us per launch (f32, split): 56, 41 at 4096 worlds, 122, 79 at
-// 65536, 241, 165 at 131072, there with the two-wave build's parked tiles and
-// priorities 161. What bounds the large launch now is VALU issue and MFMA
-// together: 8300 VALU instructions (the normals' f64, tanh, the split) and
-// 34000 cycles of MFMA per wave, which the two waves of a SIMD overlap by
-// little.
+// sign, 0.05-1.01 with equal activations of that kind too. Six 16x16x32 bf16
+// MFMAs (16 cycles each) replace eight 16x16x4 f32 ones (32 cycles each) per
+// 32 inputs: 96 against 256 cycles of matrix core, for 5.5 more VALU
+// instructions per activation. 29-256-256-8 in one wave per tile, us per
+// launch at steady clocks (f32, split): 56, 38 at 4096 worlds, 112, 71 at
+// 65536, 215, 139 at 131072, the large two in the build for two waves per SIMD
+// (154 at 131072 without its parked tiles). What bounds the large launch now
+// is VALU issue and MFMA together: 8300 VALU instructions (the normals' f64,
+// tanh, the split) and 34000 cycles of MFMA per wave, which keep the matrix
+// cores busy 49% of the launch; the two waves of a SIMD overlap by little.
 // Taken where every weight of the two layers is zero or of magnitude in
 // [2^-100, 2^100] (the host checks on upload), so that none of its pieces
 // overflows or is subnormal. Their inputs are tanh values, at most 1; of one
@@ -544,7 +545,8 @@ template <class P, class T> __device__ __forceinline__ void policy_wave(const Po
   // Two-wave builds: the second wave of a SIMD issues first where both can, so
   // that the two leave lockstep and one's VALU phases fall into the other's
   // MFMAs (workgroups fill a SIMD's first wave, then its second; the order is
-  // no more than a hint): 149 -> 145 us at 131072 worlds.
+  // no more than a hint): 71.9 -> 71.2 us at 65536 worlds, 138-142 either way
+  // at 131072, and 100 -> 52 B of spills per lane.
   if constexpr (P::PARK > 0) {
     if ((blockIdx.x >> 10) & 1) __builtin_amdgcn_s_setprio(3);
   }
@@ -641,8 +643,8 @@ template <class P, class T> __device__ __forceinline__ void policy_wave(const Po
 
 // ── small launches: a tile of 16 CB worlds to a workgroup of TW waves ──
 // One wave per tile leaves most SIMDs idle when a launch has few tiles, and
-// the launch then lasts as long as one wave's stream (29-256-256-8: 40 us at
-// 64 worlds, 44 at 16384; here 16 and 29). Here wave k computes the hidden neurons of blocks
+// the launch then lasts as long as one wave's stream (29-256-256-8: 38 us at
+// 64 worlds, 42 at 16384; here 16 and 29). Here wave k computes the hidden neurons of blocks
 // k * BPW .. of both hidden layers for the whole tile, and passes them to the
 // others through LDS, already split into bf16 pieces and laid out as B
 // fragments. The streams' raw draws are one lane's work per world, the

@@ -371,7 +371,9 @@ Plan plan_partition(const ModelD& m, const Features& f) {
   // dropped, no plan of exactly three groups), as group -> part indices.
   auto pack = [&](int cap) {
     const int n = (int)parts.size();
-    cap = std::min(cap, n);  // more groups than parts are empty ones: the same plans
+    // More groups than parts are empty ones. (Six parts are thereby searched
+    // exhaustively, 6^6 assignments, not by the greedy order of 8^6.)
+    cap = std::min(cap, n);
     std::vector<std::vector<int>> best;
     double best_cost = -1;
     auto consider = [&](const std::vector<int>& owner) {
@@ -1355,8 +1357,8 @@ std::string gen_policy_source(const PolicyD& p, int npd, bool f64, bool two_wave
   s += kControlSrc;
   const int cb = team ? team : p.cb();
   // Two-wave builds park tiles of layer 1 in LDS, up to 16 KB per wave (8
-  // waves of 18 KB a CU) instead of spilling them: at hidden 256, 284 -> 52 B
-  // of scratch per lane, 155 -> 149 us.
+  // waves of 18 KB a CU) instead of spilling them: at hidden 256, 328 -> 52 B
+  // of scratch per lane, 154 -> 139 us at 131072 worlds, 79 -> 71 at 65536.
   const int park = two_waves && p.split ? std::min(16 / cb, p.nhb() - 2) : 0;
   const int lds = std::max(16 * cb * std::max(16 * p.ku() + 1, 16 * p.nob() + 1), park * cb * 256);
   std::ostringstream o;
@@ -1602,8 +1604,9 @@ struct phz_sim {
   // Pageable hipMemcpys of f64 rows did 8-17 GB/s on readback (less into
   // memory not yet touched) and 30 GB/s on upload; this host core converts at
   // about 80 GB/s from and to cache. us per call, copies / slots: readback of
-  // 65536 x 14 f32 values 1767 / 168 (into touched memory 451 / 165), of
-  // 131072 x 28 3355 / 1644 (1653 / 690), of 8192 x 28 144 / 59, of 96 x 4 f64
+  // 65536 x 14 f32 values into fresh memory 1080 / 470 on one machine, 1680 /
+  // 1010 on another, into touched memory 650 / 220 and 710 / 330; of 131072 x
+  // 28 3355 / 1644 (touched 1653 / 690), of 8192 x 28 144 / 59, of 96 x 4 f64
   // 52 / 16; load of 65536 x 21 371 / 231, of 96 x 6 29 / 20. Small rows gain
   // from one launch and one wait for q and v together, large ones from the
   // bytes; where the caller's memory is untouched its page faults remain.
@@ -1934,11 +1937,12 @@ struct phz_sim {
       // SIMD, and its per-world VALU work (the normals, tanh) then does not
       // overlap the matrix cores. With more waves than SIMDs, a build for
       // two resident waves per SIMD (the same build: the same bits) overlaps
-      // one wave's VALU work with another's MFMAs: on the ant control workload
-      // (131072 worlds, 4096 waves) 0.255 -> 0.224 ms per launch with 164 B
-      // of spills per lane, rollout 16.99 -> 15.35 ms (all in f32; the split
-      // layers' figures are with tanh_layer_split). Taken while it spills
-      // at most 512 B per lane; PHZ_TWO_WAVES=0 keeps one wave per SIMD.
+      // one wave's VALU work with another's MFMAs. us per launch, one wave /
+      // two: 29-256-256-8 123 / 106 at 65600 worlds, 181 / 160 at 131072 (52 B
+      // of spills per lane), hidden 192 93 / 80 and 142 / 128 (168 B), 144 86 /
+      // 74 and 95 / 87 (260 B), 128 77 / 62 and 85 / 69 (20 B), each after an
+      // idle clock. Taken while it spills at most 512 B per lane;
+      // PHZ_TWO_WAVES=0 keeps one wave per SIMD.
       const char* tw = std::getenv("PHZ_TWO_WAVES");
       const long waves = ((long)nworld + 16L * pol.cb() - 1) / (16L * pol.cb());
       const int64_t regs = remark_value(k.code->log, "VGPRs:") + std::max<int64_t>(remark_value(k.code->log, "AGPRs:"), 0);
@@ -2615,7 +2619,7 @@ int phz_readback_states(phz_sim* s, double* q, double* v) {
   return s->move_rows(false, rows, 2, 1, s->f64, "readback states") ? 0 : 1;
 }
 // phz_readback_states through the library's static per-GPU scratch array
-// instead of the sim's staging buffer: no device allocation on any call.
+// instead of the sim's pinned slots: no allocation on any call.
 int phz_readback_states_noalloc(phz_sim* s, double* q, double* v) {
   if (!s) return 1;
   if (!s->has_device()) return s->fail("host-only sim has no device buffers");

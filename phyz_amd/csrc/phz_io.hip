@@ -22,12 +22,11 @@ namespace {
 // World-major rows against structure-of-arrays columns, a tile of 64 worlds x
 // 64 columns through LDS so that both sides are read and written in whole
 // lines; one grid row per part, so q, v and ctrl are one launch. The rows are
-// pinned host memory (RowsArgs in phz_host.cpp), which the kernels access over
+// pinned host memory (move_rows in phz_host.cpp), which the kernels access over
 // PCIe themselves: no device staging, no copy command, half the bytes where
 // the sim is f32. Bound by PCIe in large launches and by the launch itself in
 // small ones. The lane-per-world form read and wrote rows 8 bytes a lane, a
-// row's pitch apart, in f64; calls before and after are with move_rows in
-// phz_host.cpp.
+// row's pitch apart, in f64; calls before and after are with move_rows.
 constexpr int kTile = 64;
 
 // rows[w][c] = (R) soa[c][first + w]
