@@ -1682,11 +1682,11 @@ struct phz_sim {
     int ng = 1;
     feat.lane_small_tree = false;
     std::string src = gen_source(model, feat, f64, &ng, &lanes);
-    const double speedup = plan_partition(model, feat).speedup;
-    if (speedup > 0 && feat.wgs > feat.cus) {
+    if (ng > 1 && model.nb < 14 && !f64 && feat.wgs > feat.cus) {
+      const double speedup = plan_partition(model, feat).speedup;  // 0: not a small floating tree
       std::string e2;
       const auto co = compile_source(src, Build::Reassoc, e2);
-      if (co && !small_tree_pays(co->log, ng, speedup)) {
+      if (co && speedup > 0 && !small_tree_pays(co->log, ng, speedup)) {
         feat.lane_small_tree = true;
         src = gen_source(model, feat, f64, &ng, &lanes);
       }
