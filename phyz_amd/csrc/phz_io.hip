@@ -20,32 +20,33 @@ struct PhzRowParts {  // must match phz_host.cpp
 namespace {
 
 // World-major rows against structure-of-arrays columns, a tile of 64 worlds x
-// 64 columns through LDS so that both sides are read and written in whole
-// lines; one grid row per part, so q, v and ctrl are one launch. The rows are
-// pinned host memory (move_rows in phz_host.cpp), which the kernels access over
-// PCIe themselves: no device staging, no copy command, half the bytes where
-// the sim is f32. Bound by PCIe in large launches and by the launch itself in
-// small ones. The lane-per-world form read and wrote rows 8 bytes a lane, a
-// row's pitch apart, in f64; calls before and after are with move_rows.
+// 64 columns per workgroup through LDS so that both sides are read and written
+// in whole lines; one grid row per part, so q, v and ctrl are one launch, one
+// grid layer per column tile: a slot of wide rows holds few worlds (two tiles
+// of 64 at 1056 values), and their columns in one workgroup's turn left PCIe
+// idle. The rows are pinned host memory (move_rows in phz_host.cpp), which the
+// kernels access over PCIe themselves: no device staging, no copy command,
+// half the bytes where the sim is f32. Bound by PCIe in large launches and by
+// the launch itself in small ones. The lane-per-world form read and wrote rows
+// 8 bytes a lane, a row's pitch apart, in f64; calls before and after are with
+// move_rows.
 constexpr int kTile = 64;
 
 // rows[w][c] = (R) soa[c][first + w]
 template <class T, class R> __global__ void __launch_bounds__(256) rows_out(PhzRowParts p) {
   __shared__ T tile[kTile][kTile + 1];
   const int width = p.width[blockIdx.y], w0 = blockIdx.x * kTile, nw = min(kTile, p.count - w0);
+  const int c0 = blockIdx.z * kTile, nc = min(kTile, width - c0);
+  if (nc <= 0) return;  // a narrower part
   const T* soa = (const T*)p.soa[blockIdx.y] + p.first + w0;
   R* rows = (R*)p.rows[blockIdx.y] + (size_t)w0 * width;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  for (int c0 = 0; c0 < width; c0 += kTile) {
-    const int nc = min(kTile, width - c0);
-    if (lane < nw)
-      for (int c = wave; c < nc; c += 4) tile[lane][c] = soa[(size_t)(c0 + c) * p.stride + lane];
-    __syncthreads();
-    for (int k = threadIdx.x; k < nw * nc; k += 256) {
-      const int w = k / nc, c = k - w * nc;
-      rows[(size_t)w * width + c0 + c] = (R)tile[w][c];
-    }
-    __syncthreads();
+  if (lane < nw)
+    for (int c = wave; c < nc; c += 4) tile[lane][c] = soa[(size_t)(c0 + c) * p.stride + lane];
+  __syncthreads();
+  for (int k = threadIdx.x; k < nw * nc; k += 256) {
+    const int w = k / nc, c = k - w * nc;
+    rows[(size_t)w * width + c0 + c] = (R)tile[w][c];
   }
 }
 
@@ -53,21 +54,26 @@ template <class T, class R> __global__ void __launch_bounds__(256) rows_out(PhzR
 template <class T> __global__ void __launch_bounds__(256) rows_in(PhzRowParts p) {
   __shared__ T tile[kTile][kTile + 1];
   const int width = p.width[blockIdx.y], w0 = blockIdx.x * kTile, nw = min(kTile, p.count - w0);
+  const int c0 = blockIdx.z * kTile, nc = min(kTile, width - c0);
+  if (nc <= 0) return;
   T* soa = (T*)p.soa[blockIdx.y] + p.first + w0;
   const T* rows = (const T*)p.rows[blockIdx.y] + (size_t)w0 * width;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  for (int c0 = 0; c0 < width; c0 += kTile) {
-    const int nc = min(kTile, width - c0);
 #pragma unroll 4
-    for (int k = threadIdx.x; k < nw * nc; k += 256) {
-      const int w = k / nc, c = k - w * nc;
-      tile[w][c] = rows[(size_t)w * width + c0 + c];
-    }
-    __syncthreads();
-    if (lane < nw)
-      for (int c = wave; c < nc; c += 4) soa[(size_t)(c0 + c) * p.stride + lane] = tile[lane][c];
-    __syncthreads();
+  for (int k = threadIdx.x; k < nw * nc; k += 256) {
+    const int w = k / nc, c = k - w * nc;
+    tile[w][c] = rows[(size_t)w * width + c0 + c];
   }
+  __syncthreads();
+  if (lane < nw)
+    for (int c = wave; c < nc; c += 4) soa[(size_t)(c0 + c) * p.stride + lane] = tile[lane][c];
+}
+
+// One workgroup per tile of worlds, part and tile of columns.
+dim3 rows_grid(const PhzRowParts* p) {
+  int width = 1;
+  for (int k = 0; k < p->parts; k++) width = width > p->width[k] ? width : p->width[k];
+  return dim3((p->count + kTile - 1) / kTile, p->parts, (width + kTile - 1) / kTile);
 }
 
 template <class T> __global__ void fill_zero(T* __restrict__ dst, size_t n) {
@@ -121,7 +127,7 @@ extern "C" {
 // soa_f64, rows_f64: the element types; rows of a f32 array may be f64.
 hipError_t phz_io_rows_out(const PhzRowParts* p, int soa_f64, int rows_f64, hipStream_t s) {
   if (p->count <= 0 || p->parts <= 0) return hipSuccess;
-  const dim3 grid((p->count + kTile - 1) / kTile, p->parts), block(256);
+  const dim3 grid = rows_grid(p), block(256);
   if (soa_f64 && rows_f64) hipLaunchKernelGGL(HIP_KERNEL_NAME(rows_out<double, double>), grid, block, 0, s, *p);
   else if (soa_f64) return hipErrorInvalidValue;
   else if (rows_f64) hipLaunchKernelGGL(HIP_KERNEL_NAME(rows_out<float, double>), grid, block, 0, s, *p);
@@ -131,7 +137,7 @@ hipError_t phz_io_rows_out(const PhzRowParts* p, int soa_f64, int rows_f64, hipS
 
 hipError_t phz_io_rows_in(const PhzRowParts* p, int f64, hipStream_t s) {
   if (p->count <= 0 || p->parts <= 0) return hipSuccess;
-  const dim3 grid((p->count + kTile - 1) / kTile, p->parts), block(256);
+  const dim3 grid = rows_grid(p), block(256);
   if (f64) hipLaunchKernelGGL(rows_in<double>, grid, block, 0, s, *p);
   else hipLaunchKernelGGL(rows_in<float>, grid, block, 0, s, *p);
   return hipGetLastError();

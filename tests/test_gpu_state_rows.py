@@ -11,7 +11,7 @@ import pytest
 import torch
 
 from phyz_amd import workloads as W
-from phyz_amd.sim import from_control_loop, from_workload
+from phyz_amd.sim import BatchSim, from_control_loop, from_workload
 
 pytestmark = pytest.mark.gpu
 
@@ -60,6 +60,24 @@ def test_wide_rows(prec):
     rng = np.random.default_rng(3)
     cs = rng.normal(size=(n, nb, 56))
     ext = rng.normal(size=(n, nb, 6))
+    sim.load_contact_state(cs, ext)
+    cs2, ext2 = sim.readback_contact_state()
+    assert np.array_equal(_bits(cs2[..., 8:]), _bits(_rounded(cs[..., 8:], prec)))
+    assert np.array_equal(_bits(ext2), _bits(_rounded(ext, prec)))
+    sim.close()
+
+
+@pytest.mark.parametrize("prec", ["f32", "f64"])
+@pytest.mark.parametrize("n", [65, 300])
+def test_rows_of_many_column_tiles(n, prec):
+    """A 22-body tree's impulses are 1056 values a world, 16.5 column tiles, and
+    a full slot holds one or two tiles of worlds; 300 worlds take several."""
+    w = W.config(4)
+    sim = BatchSim(w.model, n, prec)
+    sim.enable_contact_impulse(w.contact.ground_height, w.contact.friction, w.contact_gains(), None, None)
+    rng = np.random.default_rng(n)
+    cs = rng.normal(size=(n, sim.nb, 56))
+    ext = rng.normal(size=(n, sim.nb, 6))
     sim.load_contact_state(cs, ext)
     cs2, ext2 = sim.readback_contact_state()
     assert np.array_equal(_bits(cs2[..., 8:]), _bits(_rounded(cs[..., 8:], prec)))
