@@ -1893,7 +1893,10 @@ struct phz_sim {
   // blocks per wave of 4) take the 16-world tile, whose small workgroups share
   // a CU, up to six columns per CU (five at 32, whose one-wave form is as
   // short), and wider ones the 32-world tile up to four (at five 29-160-8
-  // would still gain, 29-200-8 and the wider ones lose: 35.1 40.5 37.8).
+  // would still gain, 29-200-8 and the wider ones lose: 35.1 40.5 37.8). The
+  // widest nets (above 64 inputs, 128 neurons and 16 actions) keep 32 worlds a
+  // block at every size, as control_kernel_info has always reported for them;
+  // up to one column per CU that costs 4-6%.
   // us per launch, one wave per tile / 16-world / 32-world tiles, at 64, 4096,
   // 8192, 12288, 16384, 20480 and 24576 worlds (256 columns are 4096):
   //   29-32-8    20.7 10.9 12.3, 20.7 11.6 13.0, 21.0 13.4 13.4, 21.2 13.8 15.9,
@@ -1919,6 +1922,7 @@ struct phz_sim {
     const long columns = ((long)nworld + 15) / 16, cus = std::max(feat.cus, 1);
     const bool wide = pol.nhb() > 8;
     if (columns > cus * (wide ? 4 : pol.nhb() > 2 ? 6 : 5)) return 0;
+    if (wide && pol.n_in > 64 && pol.nob() > 1) return 2;
     return columns > cus && (wide || columns <= 2 * cus) ? 2 : 1;
   }
   // Compile (and with `load`, load) the FK/observation or the policy kernel

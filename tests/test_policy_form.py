@@ -31,7 +31,9 @@ def _form(n_in, hidden, n_out, n):
     ((29, 128, 8), (1, 1, 2, 2, 1, 1, 1, 0)),
     ((29, 129, 8), (1, 1, 2, 2, 2, 0, 0, 0)),
     ((29, 256, 8), (1, 1, 2, 2, 2, 0, 0, 0)),
-    ((128, 256, 32), (1, 1, 2, 2, 2, 0, 0, 0)),  # 36.5 us at 4096 in 16-world tiles, 38.0 in 32-world ones
+    ((128, 256, 8), (1, 1, 2, 2, 2, 0, 0, 0)),   # 30.0 us at 4096 in 16-world tiles, 31.8 in 32-world ones
+    ((60, 256, 32), (1, 1, 2, 2, 2, 0, 0, 0)),
+    ((128, 256, 32), (2, 2, 2, 2, 2, 0, 0, 0)),  # 32 worlds a block at every size (36.5 us at 4096 in 16, 38.0)
 ])
 def test_form_by_size(shape, forms, monkeypatch):
     monkeypatch.delenv("PHZ_POLICY_TEAM", raising=False)
