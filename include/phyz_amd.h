@@ -151,7 +151,7 @@ int phz_readback_states(phz_sim* sim, double* q, double* v);
 /* No counterpart in the reference. For callers that cannot allocate device
  * memory (tight serving loops, harnesses that forbid hipMalloc):
  * phz_readback_states staged through the library's static 32 MiB per-GPU
- * scratch array instead of the sim's lazily allocated pinned slots, so no
+ * scratch array instead of the sim's own pinned slots, so no
  * call allocates. Rejects nworld * max(nq, nv) * 8 bytes above 32 MiB.
  * Synchronizes the sim's stream, so it returns an error while that stream is
  * capturing a graph. All calls on one GPU share its array and take turns on a
